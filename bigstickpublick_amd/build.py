@@ -17,16 +17,32 @@ HIP_FLAGS = [
 ]
 
 
+SOURCES = ("bs_engine.hip", "bs_like.hip", "bs_tables.cpp")
+
+
 def build_native(verbose=False):
-    srcs = [os.path.join(CSRC, "bs_engine.hip"), os.path.join(CSRC, "bs_tables.cpp")]
+    """Compiles every source (side by side) and links the library."""
+    bdir = os.path.join(CSRC, "_build")
+    os.makedirs(bdir, exist_ok=True)
+    inc = ["-I", os.path.join(os.path.dirname(HERE), "include")]
+    jobs = []
+    for src in SOURCES:
+        obj = os.path.join(bdir, src + ".o")
+        cmd = [HIPCC] + [f for f in HIP_FLAGS if f != "-shared"] + inc + ["-c", os.path.join(CSRC, src), "-o", obj]
+        jobs.append((obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+    for obj, p in jobs:
+        out = p.communicate()[0]
+        if p.returncode != 0:
+            for _, q in jobs:
+                q.wait()
+            raise RuntimeError("hipcc failed:\n" + out)
+        if verbose:
+            print(out)
     tmp = LIB + ".tmp"
-    cmd = [HIPCC] + HIP_FLAGS + ["-I", os.path.join(os.path.dirname(HERE), "include"),
-                                 "-o", tmp] + srcs + ["-lrocsolver", "-lrocblas"]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-o", tmp] + [obj for obj, _ in jobs] +
+                       ["-lrocsolver", "-lrocblas"], capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed:\n" + r.stdout + r.stderr)
-    if verbose:
-        print(r.stderr)
     os.replace(tmp, LIB)
     return LIB
 

@@ -34,6 +34,7 @@
 
 #include "../../include/bigstick_amd.h"
 #include "bs_tables.hpp"
+#include "bs_like.hpp"
 #include <rocsolver/rocsolver.h>
 #include <atomic>
 #include <mutex>
@@ -68,6 +69,7 @@ struct DevTables {
   int64_t dim;
   int nP, nN, ndelta;
   int call_spe;
+  int like;                  // include SPE, PP and NN
   int lmax;                  // longest neutron row
   int wcols;                 // LDS row stride of the pn element block (max class size + 1)
   const int64_t* pstart;     // [nP] row offset of proton SD
@@ -260,6 +262,16 @@ __global__ __launch_bounds__(BLOCK, PF ? 4 : 1) void k_apply_tiles(DevTables tb,
 #pragma unroll
     for (int q = 0; q < CPT; q++) acc[r][q] = T(0);
 
+  if (!tb.like) {
+    // PP and NN came before (bs_like.hip): the sum goes on from y
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < nr) {
+        const int64_t bf = tb.pstart[f0 + r];
+#pragma unroll
+        for (int q = 0; q < CPT; q++) acc[r][q] = y[bf + cl[q]];
+      }
+  } else {
   // ---- SPE (only when the single-particle energies are not subsumed)
   if (tb.call_spe) {
 #pragma unroll
@@ -363,6 +375,7 @@ __global__ __launch_bounds__(BLOCK, PF ? 4 : 1) void k_apply_tiles(DevTables tb,
         for (int r = 0; r < R; r++) acc[r][q] = fma(v[q], xv.v[r], acc[r][q]);
       }
     }
+  }
   }
   // ---- PN: per Delta class, batches of G source rows staged transposed
   const int gsel = G == 1 ? 0 : (G == 2 ? 1 : 2);
@@ -667,7 +680,7 @@ __global__ __launch_bounds__(BLOCK, PF ? 4 : 1) void k_apply_tiles(DevTables tb,
       for (int q = 0; q < CPT; q++) {
         const int c = tid + q * BLOCK;
         if (c < L) {
-          if (accumulate) y[bf + c] += acc[r][q];
+          if (accumulate && tb.like) y[bf + c] += acc[r][q];
           else y[bf + c] = acc[r][q];
         }
       }
@@ -2352,7 +2365,7 @@ struct bs_system {
   DevBuf<int32_t> rows_f, rows_c;  // k_apply_rows: (proton row, first column) per workgroup
   int nrows_wg = 0;
   int variant[2] = {-1, -1};   // chosen kernel variant per dtype (0: f32, 1: f64)
-  float tune_ms[2][32] = {};    // autotuner timings (ms; 0 = not run / does not fit)
+  float tune_ms[2][64] = {};    // autotuner timings (ms; 0 = not run / does not fit)
   DevTables dt{};
   DevBuf<int64_t> pstart, pp_ptr, nn_base, n1_base, n1q_base;
   DevBuf<int32_t> tile_f0[3], tile_nr[3], tile_map[3][2];
@@ -2370,6 +2383,7 @@ struct bs_system {
   DevBuf<uint32_t> n1_pkr;
   DevBuf<float> pspe_sd, nspe_sd, pp_val32, nn_val32, W;
   DevBuf<double> pp_val64, nn_val64;
+  bsl::Owner like;              // tables of the separate PP and NN kernels
 };
 
 namespace {
@@ -2784,6 +2798,7 @@ void upload_tables(bs_system* s) {
   d.nN = nN;
   d.ndelta = nd;
   d.call_spe = t.call_spe ? 1 : 0;
+  d.like = 1;
   d.lmax = lmax;
   d.wcols = t.max_class + 1;
   d.pstart = s->pstart.p;
@@ -2819,6 +2834,7 @@ void upload_tables(bs_system* s) {
   d.wrows = s->wrows.p;
   d.wstride = s->wstride.p;
   d.negk = s->negk.p;
+  if (s->tiles_ok) bsl::build(s->like, t, s->pstart.p, s->psec.p, s->pconj.p, s->nlen.p, nlen, s->pp_ptr.p, s->pp_src.p, s->pp_val64.p);
   s->uploaded = true;
 }
 
@@ -2840,8 +2856,9 @@ size_t lds_bytes(const bs_system* s, int v);
 
 constexpr size_t kLdsLimit = 160 * 1024;
 
+// like = false: the proton-neutron part only
 template <typename T, int CPT, int R, int G>
-void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumulate, hipStream_t st) {
+void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumulate, hipStream_t st, bool like = true) {
   const int ri = R == 1 ? 0 : (R == 2 ? 1 : 2);
   DevTables d = s->dt;
   d.tile_f0 = s->tile_f0[ri].p;
@@ -2851,6 +2868,7 @@ void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumu
   d.tpp_src = s->tpp_src[ri].p;
   d.tpp_val32 = s->tpp_val32[ri].p;
   d.tpp_val64 = s->tpp_val64[ri].p;
+  d.like = like;
   // static LDS (lds_bytes_rg).  Where it leaves room for one workgroup per
   // CU only (FP64 with four staged rows: 132 KB), the workgroup has 1024
   // threads with half the columns each, so a CU still holds 16 waves; every
@@ -2871,29 +2889,45 @@ void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumu
   HIP_OK(hipGetLastError());
 }
 
-// the row kernel, after the tile variants
-constexpr int kRowsVariant = kNumVariants;
-constexpr int kAllVariants = kNumVariants + 1;
+// After the tile variants: PP and NN by their own kernels (bs_like.hip) with
+// the proton-neutron part by each tile shape (XCD map, PF), and the row kernel.
+// The separate kernels read a PP source row once per 16 target rows on the
+// matrix cores and an NN entry once per 8 rows, which the tile kernel's LDS and
+// registers have no room for (pf 6p6n: 2.9 + 1.5 ms FP32, 5.4 + 2.8 ms FP64).
+// They pay from rows of some hundred columns on (pf 4p4n FP32 549 -> 464 us,
+// pf 6p6n 21.0 -> 18.9 ms, FP64 42.7 -> 35.2 ms); on short rows the two extra
+// launches and the tiles' padding cost more (pf 2p3n 32 -> 68 us).
+constexpr int kLikeVariant = kNumVariants;
+constexpr int kRowsVariant = kLikeVariant + kNumShapes;
+constexpr int kAllVariants = kRowsVariant + 1;
+constexpr int64_t kLikeDim = 1000000;  // basis size from which they are the default
+constexpr bool is_like(int v) { return v >= kLikeVariant && v < kRowsVariant; }
 
 template <typename T>
 size_t lds_bytes(const bs_system* s, int v) {
   if (v == kRowsVariant) return 0;
   if (!s->tiles_ok) return SIZE_MAX;
+  if (is_like(v) && !s->like.ok) return SIZE_MAX;
   return lds_bytes_rg<T>(s, kVarR[v % kNumShapes], kVarG[v % kNumShapes]);
 }
 
 template <typename T, int CPT>
 void launch_cpt(bs_system* s, int v, const T* x, T* y, int accumulate, hipStream_t st) {
-  const int m = (v / kNumShapes) % 2;
+  const bool like = is_like(v);
+  const int m = like ? 1 : (v / kNumShapes) % 2;
   const bool pf = v >= 2 * kNumShapes;
+  if (like) {
+    bsl::apply(s->like, x, y, accumulate, st);
+    accumulate = 1;
+  }
   switch (v % kNumShapes) {
-    case 0: launch_variant<T, CPT, 1, 1>(s, m, pf, x, y, accumulate, st); break;
-    case 1: launch_variant<T, CPT, 1, 2>(s, m, pf, x, y, accumulate, st); break;
-    case 2: launch_variant<T, CPT, 2, 1>(s, m, pf, x, y, accumulate, st); break;
-    case 3: launch_variant<T, CPT, 2, 2>(s, m, pf, x, y, accumulate, st); break;
-    case 4: launch_variant<T, CPT, 2, 4>(s, m, pf, x, y, accumulate, st); break;
-    case 5: launch_variant<T, CPT, 4, 2>(s, m, pf, x, y, accumulate, st); break;
-    default: launch_variant<T, CPT, 4, 4>(s, m, pf, x, y, accumulate, st); break;
+    case 0: launch_variant<T, CPT, 1, 1>(s, m, pf, x, y, accumulate, st, !like); break;
+    case 1: launch_variant<T, CPT, 1, 2>(s, m, pf, x, y, accumulate, st, !like); break;
+    case 2: launch_variant<T, CPT, 2, 1>(s, m, pf, x, y, accumulate, st, !like); break;
+    case 3: launch_variant<T, CPT, 2, 2>(s, m, pf, x, y, accumulate, st, !like); break;
+    case 4: launch_variant<T, CPT, 2, 4>(s, m, pf, x, y, accumulate, st, !like); break;
+    case 5: launch_variant<T, CPT, 4, 2>(s, m, pf, x, y, accumulate, st, !like); break;
+    default: launch_variant<T, CPT, 4, 4>(s, m, pf, x, y, accumulate, st, !like); break;
   }
 }
 
@@ -2934,6 +2968,9 @@ int autotune(bs_system* s, hipStream_t st) {
   int bestv = -1;
   for (int v = 0; v < kAllVariants; v++) {
     if (lds_bytes<T>(s, v) > kLdsLimit) continue;
+    // on large bases the staged-after tiles never won against the PF ones
+    // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
+    if (v < 2 * kNumShapes && s->like.ok && D >= kLikeDim) continue;
     launch_apply_v<T>(s, v, x.p, y.p, 0, st);
     HIP_OK(hipEventRecord(e0, st));
     launch_apply_v<T>(s, v, x.p, y.p, 0, st);
@@ -2955,8 +2992,9 @@ template <typename T>
 void launch_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st) {
   const int di = sizeof(T) == 4 ? 0 : 1;
   if (s->variant[di] < 0) {
-    // default: the largest tile that fits, until autotuned
-    int v = 2 * kNumShapes - 1;
+    // until autotuned: the largest tile that fits, on large bases with the
+    // separate PP and NN kernels
+    int v = s->like.ok && s->t.dim >= kLikeDim ? kRowsVariant - 1 : 2 * kNumShapes - 1;
     while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
     s->variant[di] = v >= 0 ? v : kRowsVariant;
   }
@@ -4857,8 +4895,8 @@ int bs_variant_info(int v, int* rows, int* staged, int* xcd_map, int* prefetch) 
   }
   if (rows) *rows = kVarR[v % kNumShapes];
   if (staged) *staged = kVarG[v % kNumShapes];
-  if (xcd_map) *xcd_map = (v / kNumShapes) % 2;
-  if (prefetch) *prefetch = v >= 2 * kNumShapes;
+  if (xcd_map) *xcd_map = is_like(v) ? 1 : (v / kNumShapes) % 2;
+  if (prefetch) *prefetch = is_like(v) ? 2 : v >= 2 * kNumShapes;
   return 0;
 }
 

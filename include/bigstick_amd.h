@@ -118,7 +118,9 @@ int bs_apply_h(bs_system *sys, const void *x, void *y, int dtype, int accumulate
  * workgroup-to-tile order (xcd_map 0: sector order; 1: runs of consecutive
  * tiles on the workgroups that the dispatcher places on one XCD, so each
  * XCD's L2 holds their shared source rows), and prefetch (1: the next batch
- * of source rows is loaded into registers while the current one is applied).
+ * of source rows is loaded into registers while the current one is applied;
+ * 2: the same, with the proton-proton and neutron-neutron parts by kernels of
+ * their own).
  * The last variant (staged = 0) is the row kernel: one thread per output
  * state, every gather from global memory, no LDS; it is the only one on
  * spaces whose neutron sectors exceed 4096 SDs or whose Delta-m operator
