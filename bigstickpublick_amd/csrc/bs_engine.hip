@@ -1880,13 +1880,39 @@ __global__ __launch_bounds__(256) void k_bmultidot(const T* __restrict__ V, int6
   }
 }
 
-// out[j*K + k] = sum_b part[...]; mode 1: sqrt
-__global__ void k_breduce(const double* __restrict__ part, int nb, int m, int K, double* __restrict__ out, int mode) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= m * K) return;
+// out[j*K + k] = sum_b part[b][j][k] (workgroup j; mode 1: its square root).
+// Lane = Hamiltonian, the partial sums of the up to 512 blocks spread over 16
+// waves with eight loads each in flight: one thread walking them all waits out
+// a memory latency per block (446 blocks: 107 us, here 6).
+constexpr int kBReduce = 1024;
+__device__ __forceinline__ void breduce(const double* __restrict__ part, int nb, int m, int K, double* __restrict__ out,
+                                        int mode) {
+  __shared__ double red[kBReduce / 64][64];
+  const int k = threadIdx.x & 63, wv = threadIdx.x >> 6, j = blockIdx.x;
+  constexpr int NW = kBReduce / 64;
   double s = 0.0;
-  for (int b = 0; b < nb; b++) s += part[(int64_t)b * m * K + idx];
-  out[idx] = mode == 1 ? sqrt(s) : s;
+  if (k < K) {
+    const double* p = part + (int64_t)j * K + k;
+    const int64_t st = (int64_t)m * K;
+    for (int b = wv; b < nb; b += 8 * NW) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = b + u * NW < nb ? p[(b + u * NW) * st] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+  }
+  red[wv][k] = s;
+  __syncthreads();
+  if (wv == 0 && k < K) {
+    double t = 0.0;
+    for (int q = 0; q < NW; q++) t += red[q][k];
+    out[(int64_t)j * K + k] = mode == 1 ? sqrt(t) : t;
+  }
+}
+__global__ __launch_bounds__(kBReduce) void k_breduce(const double* __restrict__ part, int nb, int m, int K,
+                                                      double* __restrict__ out, int mode) {
+  breduce(part, nb, m, K, out, mode);
 }
 
 template <typename T>
@@ -1990,14 +2016,11 @@ __global__ __launch_bounds__(256) void k_bmultidot_g(const T* __restrict__ V, in
   }
 }
 
-__global__ void k_breduce_g(const double* __restrict__ part, int nb, int m, int K, double* __restrict__ out, int mode,
-                            const int* __restrict__ flags, int minflag) {
+__global__ __launch_bounds__(kBReduce) void k_breduce_g(const double* __restrict__ part, int nb, int m, int K,
+                                                        double* __restrict__ out, int mode,
+                                                        const int* __restrict__ flags, int minflag) {
   if (flags[K] < minflag) return;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= m * K) return;
-  double s = 0.0;
-  for (int b = 0; b < nb; b++) s += part[(int64_t)b * m * K + idx];
-  out[idx] = mode == 1 ? sqrt(s) : s;
+  breduce(part, nb, m, K, out, mode);
 }
 
 // members with flag 1 keep their vector unless it overlaps a stored one by
@@ -2056,106 +2079,154 @@ __global__ void k_bnormalize_m(T* __restrict__ v, const double* __restrict__ nrm
   }
 }
 
-// Lowest nkeep eigenpairs of K symmetric tridiagonal matrices (alpha[i*K+k],
-// beta[i*K+k] = coupling of i and i+1), FP64, one thread per matrix: Sturm
-// bisection for the eigenvalues, inverse iteration (tridiagonal LU with
-// partial pivoting) for the vectors.  Y[(k*m + i)*nkeep + n].
-__global__ void k_tridiag_ritz(const double* __restrict__ alpha, const double* __restrict__ beta, int m, int K,
-                               int nkeep, double* __restrict__ evals, double* __restrict__ Y, double* __restrict__ work) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= K) return;
-  auto a = [&](int i) { return alpha[(int64_t)i * K + k]; };
-  auto b = [&](int i) { return beta[(int64_t)i * K + k]; };
-  double lo = 1e300, hi = -1e300;
-  for (int i = 0; i < m; i++) {
-    const double r = (i > 0 ? fabs(b(i - 1)) : 0.0) + (i + 1 < m ? fabs(b(i)) : 0.0);
-    lo = fmin(lo, a(i) - r);
-    hi = fmax(hi, a(i) + r);
+// Lowest nkeep (<= 16) eigenpairs of K symmetric tridiagonal matrices
+// (alpha[i*K+k], beta[i*K+k] = coupling of i and i+1), FP64, a workgroup per
+// matrix and a wave per eigenvalue.  Eigenvalues by Sturm counts at 64 points
+// of the interval at a time (one a lane: an interval shrinks 65-fold per
+// count, where bisection needs six counts, each a chain of m divisions);
+// vectors by inverse iteration (tridiagonal LU with partial pivoting), one
+// after the other by the first wave, the dots and updates over its lanes and
+// the recurrences on one.  With one thread a matrix the 64 matrices of an
+// ensemble, m = 30, took 2.6 ms.  Y[(k*m + i)*nkeep + n].
+__global__ __launch_bounds__(1024) void k_tridiag_ritz(const double* __restrict__ alpha, const double* __restrict__ beta,
+                                                       int m, int K, int nkeep, double* __restrict__ evals,
+                                                       double* __restrict__ Y, double* __restrict__ work) {
+  const int k = blockIdx.x, lane = threadIdx.x & 63, n0 = threadIdx.x >> 6;
+  __shared__ double lam_s[16];
+  double* wk = work + (int64_t)k * 8 * m;
+  double* av = wk;           // this matrix, contiguous
+  double* bv = wk + m;
+  double* dd = wk + 2 * m;   // LU diagonal
+  double* du = wk + 3 * m;   // first superdiagonal
+  double* du2 = wk + 4 * m;  // second superdiagonal (pivoting)
+  double* dl = wk + 5 * m;   // multipliers
+  int* piv = (int*)(wk + 6 * m);
+  double* v = wk + 7 * m;
+  for (int i = threadIdx.x; i < m; i += blockDim.x) {
+    av[i] = alpha[(int64_t)i * K + k];
+    bv[i] = beta[(int64_t)i * K + k];
   }
-  double* wk = work + (int64_t)k * 6 * m;
-  double* dd = wk;         // LU diagonal
-  double* du = wk + m;     // first superdiagonal
-  double* du2 = wk + 2 * m;  // second superdiagonal (pivoting)
-  double* dl = wk + 3 * m;   // multipliers
-  int* piv = (int*)(wk + 4 * m);
-  double* v = wk + 5 * m;
-  for (int n = 0; n < nkeep; n++) {
-    // count of eigenvalues below x (Sturm sequence)
+  __syncthreads();
+  double lo = 1e300, hi = -1e300;
+  for (int i = lane; i < m; i += 64) {
+    const double r = (i > 0 ? fabs(bv[i - 1]) : 0.0) + (i + 1 < m ? fabs(bv[i]) : 0.0);
+    lo = fmin(lo, av[i] - r);
+    hi = fmax(hi, av[i] + r);
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+  }
+  for (int n = n0; n < nkeep; n += blockDim.x >> 6) {
     double l = lo, h = hi;
-    for (int it = 0; it < 200 && h - l > 1e-15 * fmax(1.0, fabs(l) + fabs(h)); it++) {
-      const double x = 0.5 * (l + h);
+    for (int it = 0; it < 60 && h - l > 1e-15 * fmax(1.0, fabs(l) + fabs(h)); it++) {
+      // eigenvalues below x (Sturm sequence), x = l + (lane + 1) (h - l) / 65
+      const double step = (h - l) / 65.0;
+      const double x = l + (lane + 1) * step;
       int cnt = 0;
       double q = 1.0;
       for (int i = 0; i < m; i++) {
-        const double bb = i > 0 ? b(i - 1) : 0.0;
-        q = a(i) - x - (i > 0 ? bb * bb / q : 0.0);
+        const double bb = i > 0 ? bv[i - 1] : 0.0;
+        q = av[i] - x - (i > 0 ? bb * bb / q : 0.0);
         if (q == 0.0) q = -1e-300;
         if (q < 0.0) cnt++;
       }
-      if (cnt > n) h = x;
-      else l = x;
+      // the first point with more than n eigenvalues below bounds it from above
+      const unsigned long long above = __ballot(cnt > n);
+      const int p = above ? __builtin_ctzll(above) : 64;
+      const double nl = p > 0 ? __shfl(x, p - 1, 64) : l, nh = p < 64 ? __shfl(x, p, 64) : h;
+      if (!(nl > l) && !(nh < h)) break;  // at the spacing of the numbers
+      l = nl;
+      h = nh;
     }
-    const double lam = 0.5 * (l + h);
-    evals[(int64_t)k * nkeep + n] = lam;
+    if (lane == 0) {
+      lam_s[n] = 0.5 * (l + h);
+      evals[(int64_t)k * nkeep + n] = 0.5 * (l + h);
+    }
+  }
+  __syncthreads();
+  if (n0 > 0) return;
+  double* Yk = Y + (int64_t)k * m * nkeep;
+  for (int n = 0; n < nkeep; n++) {
     // LU of (T - lam) with partial pivoting (tridiagonal -> bandwidth 2)
+    const double lam = lam_s[n];
     const double shift = lam + 1e-13 * fmax(1.0, fabs(lam));
-    for (int i = 0; i < m; i++) {
-      dd[i] = a(i) - shift;
-      du[i] = i + 1 < m ? b(i) : 0.0;
-      du2[i] = 0.0;
-    }
-    double sub = m > 1 ? b(0) : 0.0;
-    for (int i = 0; i < m - 1; i++) {
-      const double nxt_sub = i + 2 < m ? b(i + 1) : 0.0;
-      if (fabs(dd[i]) >= fabs(sub)) {
-        piv[i] = 0;
-        const double mult = sub / (dd[i] == 0.0 ? 1e-300 : dd[i]);
-        dl[i] = mult;
-        dd[i + 1] -= mult * du[i];
-      } else {
-        piv[i] = 1;
-        const double mult = dd[i] / sub;
-        dl[i] = mult;
-        dd[i] = sub;
-        double t0 = du[i];
-        du[i] = dd[i + 1];
-        dd[i + 1] = t0 - mult * du[i];
-        du2[i] = du[i + 1];
-        du[i + 1] = -mult * du[i + 1];
-      }
-      sub = nxt_sub;
-    }
-    for (int i = 0; i < m; i++) v[i] = 1.0 / sqrt((double)m) * (1.0 + 0.01 * (double)((i * 7919) % 13));
-    for (int rep = 0; rep < 4; rep++) {
-      // forward: apply the row operations
+    for (int i = lane; i < m; i += 64) v[i] = 1.0 / sqrt((double)m) * (1.0 + 0.01 * (double)((i * 7919) % 13));
+    if (lane == 0) {
+      double d = av[0] - shift, u = m > 1 ? bv[0] : 0.0, sub = u;
       for (int i = 0; i < m - 1; i++) {
-        if (piv[i]) {
-          const double t0 = v[i];
-          v[i] = v[i + 1];
-          v[i + 1] = t0 - dl[i] * v[i];
+        const double nd = av[i + 1] - shift, nu = i + 2 < m ? bv[i + 1] : 0.0;
+        if (fabs(d) >= fabs(sub)) {
+          piv[i] = 0;
+          const double mult = sub / (d == 0.0 ? 1e-300 : d);
+          dl[i] = mult;
+          dd[i] = d;
+          du[i] = u;
+          du2[i] = 0.0;
+          d = nd - mult * u;
+          u = nu;
         } else {
-          v[i + 1] -= dl[i] * v[i];
+          piv[i] = 1;
+          const double mult = d / sub;
+          dl[i] = mult;
+          dd[i] = sub;
+          du[i] = nd;
+          du2[i] = nu;
+          d = u - mult * nd;
+          u = -mult * nu;
+        }
+        sub = nu;
+      }
+      dd[m - 1] = d;
+      du[m - 1] = u;
+      du2[m - 1] = 0.0;
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    for (int rep = 0; rep < 4; rep++) {
+      if (lane == 0) {
+        // forward: the row operations
+        double c = v[0];
+        for (int i = 0; i < m - 1; i++) {
+          const double nx = v[i + 1];
+          if (piv[i]) {
+            v[i] = nx;
+            c = c - dl[i] * nx;
+          } else {
+            v[i] = c;
+            c = nx - dl[i] * c;
+          }
+        }
+        v[m - 1] = c;
+        // back substitution
+        double x1 = 0.0, x2 = 0.0;
+        for (int i = m - 1; i >= 0; i--) {
+          double t0 = v[i];
+          if (i + 1 < m) t0 -= du[i] * x1;
+          if (i + 2 < m) t0 -= du2[i] * x2;
+          x2 = x1;
+          x1 = t0 / (dd[i] == 0.0 ? 1e-300 : dd[i]);
+          v[i] = x1;
         }
       }
-      // back substitution
-      for (int i = m - 1; i >= 0; i--) {
-        double t0 = v[i];
-        if (i + 1 < m) t0 -= du[i] * v[i + 1];
-        if (i + 2 < m) t0 -= du2[i] * v[i + 2];
-        v[i] = t0 / (dd[i] == 0.0 ? 1e-300 : dd[i]);
-      }
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
       // orthogonalize against the previous vectors of this matrix, normalize
       for (int p = 0; p < n; p++) {
         double dot = 0.0;
-        for (int i = 0; i < m; i++) dot += v[i] * Y[((int64_t)k * m + i) * nkeep + p];
-        for (int i = 0; i < m; i++) v[i] -= dot * Y[((int64_t)k * m + i) * nkeep + p];
+        for (int i = lane; i < m; i += 64) dot += v[i] * Yk[(int64_t)i * nkeep + p];
+        for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
+        for (int i = lane; i < m; i += 64) v[i] -= dot * Yk[(int64_t)i * nkeep + p];
       }
       double nrm = 0.0;
-      for (int i = 0; i < m; i++) nrm += v[i] * v[i];
+      for (int i = lane; i < m; i += 64) nrm += v[i] * v[i];
+      for (int o = 32; o > 0; o >>= 1) nrm += __shfl_xor(nrm, o, 64);
       nrm = 1.0 / sqrt(nrm);
-      for (int i = 0; i < m; i++) v[i] *= nrm;
+      for (int i = lane; i < m; i += 64) v[i] *= nrm;
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
     }
-    for (int i = 0; i < m; i++) Y[((int64_t)k * m + i) * nkeep + n] = v[i];
+    for (int i = lane; i < m; i += 64) Yk[(int64_t)i * nkeep + n] = v[i];
   }
 }
 
@@ -4365,15 +4436,15 @@ void enqueue_batch_steps(bs_batch* b, bs_batch::Work& w, int i0, int i1, hipStre
     T* vi = V + (int64_t)i * DK;
     launch_batched_chosen<T>(s, b->bv, vi, wv, st);
     k_bmultidot<T><<<nb, 256, 0, st>>>(vi, DK, 1, wv, D, K, w.part.p);
-    k_breduce<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.alpha.p + (int64_t)i * K, 0);
+    k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.alpha.p + (int64_t)i * K, 0);
     k_bsub_scaled<T><<<g, kBlock, 0, st>>>(wv, vi, w.alpha.p + (int64_t)i * K, D, K);
     if (i > 0) {
       k_bmultidot<T><<<nb, 256, 0, st>>>(V, DK, i, wv, D, K, w.part.p);
-      k_breduce<<<(i * K + 255) / 256, 256, 0, st>>>(w.part.p, nb, i, K, w.dots.p, 0);
+      k_breduce<<<i, kBReduce, 0, st>>>(w.part.p, nb, i, K, w.dots.p, 0);
       k_bmultiaxpy<T><<<g, kBlock, 0, st>>>(wv, V, DK, i, w.dots.p, D, K);
     }
     k_bmultidot<T><<<nb, 256, 0, st>>>(wv, DK, 1, wv, D, K, w.part.p);
-    k_breduce<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.beta.p + (int64_t)i * K, 1);
+    k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.beta.p + (int64_t)i * K, 1);
     // v_{i+1} with the breakdown handling of k_bbreak: random restarts
     // (flag 2) are orthonormalized against v_0..v_i twice, members whose
     // beta fell below 0.1 of the previous one (flag 1) once if they lost
@@ -4389,16 +4460,16 @@ void enqueue_batch_steps(bs_batch* b, bs_batch::Work& w, int i0, int i1, hipStre
         if (pass == 0) {
           // normalize the random vectors first
           k_bmultidot_g<T><<<nb, 256, 0, st>>>(vn, DK, 1, vn, D, K, w.part.p, w.flags.p, 2);
-          k_breduce_g<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.bnorm.p, 1, w.flags.p, 2);
+          k_breduce_g<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.bnorm.p, 1, w.flags.p, 2);
           k_bnormalize_m<T><<<g, kBlock, 0, st>>>(vn, w.bnorm.p, D, K, w.flags.p, 2);
           continue;
         }
         k_bmultidot_g<T><<<nb, 256, 0, st>>>(V, DK, m, vn, D, K, w.part.p, w.flags.p, minflag);
-        k_breduce_g<<<(m * K + 255) / 256, 256, 0, st>>>(w.part.p, nb, m, K, w.dots.p, 0, w.flags.p, minflag);
+        k_breduce_g<<<m, kBReduce, 0, st>>>(w.part.p, nb, m, K, w.dots.p, 0, w.flags.p, minflag);
         if (pass == 1) k_bloss<<<1, 64, 0, st>>>(w.dots.p, m, K, w.flags.p);
         k_bmultiaxpy_m<T><<<g, kBlock, 0, st>>>(vn, V, DK, m, w.dots.p, D, K, w.flags.p, minflag);
         k_bmultidot_g<T><<<nb, 256, 0, st>>>(vn, DK, 1, vn, D, K, w.part.p, w.flags.p, minflag);
-        k_breduce_g<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.bnorm.p, 1, w.flags.p, minflag);
+        k_breduce_g<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.bnorm.p, 1, w.flags.p, minflag);
         k_bnormalize_m<T><<<g, kBlock, 0, st>>>(vn, w.bnorm.p, D, K, w.flags.p, minflag);
       }
     }
@@ -4503,7 +4574,7 @@ __global__ void k_copy(T* __restrict__ dst, const T* __restrict__ src, int64_t n
 void enqueue_batch_ritz(bs_batch::Work& w, int K, int kstart, int nout, hipStream_t st) {
   const int m = w.niter;
   if (kstart == 0 && w.thick == 0) {
-    k_tridiag_ritz<<<(K + 63) / 64, 64, 0, st>>>(w.alpha.p, w.beta.p, m, K, nout, w.evals.p, w.Y.p, w.tdwork.p);
+    k_tridiag_ritz<<<K, 64 * nout, 0, st>>>(w.alpha.p, w.beta.p, m, K, nout, w.evals.p, w.Y.p, w.tdwork.p);
   } else {
     k_projected<<<dim3((m * m + 255) / 256, K), 256, 0, st>>>(w.alpha.p, w.beta.p, w.arrow.p, kstart, m, K, w.A.p);
     k_jacobi_ritz<<<(K + 63) / 64, 64, 0, st>>>(w.A.p, m, K, nout, w.evals.p, w.Y.p, w.tdwork.p);
@@ -4543,15 +4614,15 @@ void enqueue_batch_finish(bs_batch* b, bs_batch::Work& w, int nout, hipStream_t 
   for (int q = 0; q < nkeep; q++) {
     double* xq = X + (int64_t)q * DK;
     k_bmultidot<double><<<nb, 256, 0, st>>>(xq, DK, 1, xq, D, K, w.part.p);
-    k_breduce<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.dots.p, 1);
+    k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.dots.p, 1);
     k_bnormalize<double><<<g, kBlock, 0, st>>>(xq, xq, w.dots.p, D, K);
     if (w.polish) {
       launch_batched_chosen<double>(s, b->bv, xq, HX, st);
       k_bmultidot<double><<<nb, 256, 0, st>>>(xq, DK, 1, HX, D, K, w.part.p);
-      k_breduce<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.rq.p + (int64_t)q * K, 0);
+      k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.rq.p + (int64_t)q * K, 0);
       k_bsub_scaled<double><<<g, kBlock, 0, st>>>(HX, xq, w.rq.p + (int64_t)q * K, D, K);
       k_bmultidot<double><<<nb, 256, 0, st>>>(HX, DK, 1, HX, D, K, w.part.p);
-      k_breduce<<<(K + 255) / 256, 256, 0, st>>>(w.part.p, nb, 1, K, w.res.p + (int64_t)q * K, 1);
+      k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.res.p + (int64_t)q * K, 1);
     }
   }
   HIP_OK(hipGetLastError());
@@ -4615,7 +4686,7 @@ void run_batch_lanczos(bs_batch* b, const bs_lanczos_params* p, double* alpha, d
     w.beta.alloc((size_t)niter * K);
     w.evals.alloc((size_t)K * nout);
     w.Y.alloc((size_t)K * niter * nout);
-    w.tdwork.alloc((size_t)K * std::max(6 * niter, thick ? niter * niter : 0));
+    w.tdwork.alloc((size_t)K * std::max(8 * niter, thick ? niter * niter : 0));
     w.rq.alloc((size_t)nkeep * K);
     w.res.alloc((size_t)nkeep * K);
     if (thick) w.A.alloc((size_t)K * niter * niter);
