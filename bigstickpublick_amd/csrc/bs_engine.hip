@@ -1310,6 +1310,31 @@ struct BatchVals {
   const double* kt64;
 };
 
+// Neutron one-body entries of (target sector c, class k) column by column:
+// ent[ptr[base[c*nd+k] + column] .. ptr[.. + 1]); x: source column | operator << 16
+// | negative phase << 31, y: the column | its last entry << 31
+struct LaneTables {
+  const int32_t* base;
+  const int32_t* ptr;
+  const uint2* ent;
+  int jumps;  // most of a proton row
+};
+// A class of a proton row: its jumps, coefficient row length and start, source
+// row's numbers, list of entries
+struct LaneClass {
+  int p0, p1, ws, woff, n, lp;
+};
+struct LaneLds {  // byte offsets in k_apply_lanes' LDS
+  uint32_t cls, xs, yl, wb, bytes;
+  __host__ __device__ LaneLds(int H, int G, int size, int row, int coef, int jumps, int nd) {
+    cls = (uint32_t)jumps * sizeof(uint2);
+    xs = (cls + (uint32_t)nd * sizeof(LaneClass) + 15u) & ~15u;
+    yl = xs + (uint32_t)(H * G * size) * (uint32_t)row;
+    wb = (yl + (uint32_t)size * (uint32_t)row + 15u) & ~15u;
+    bytes = wb + (uint32_t)(H * G) * (uint32_t)coef * 4u;
+  }
+};
+
 template <typename T> __device__ __forceinline__ T bval(const float* a, const double* b, int64_t i);
 template <> __device__ __forceinline__ float bval<float>(const float* a, const double*, int64_t i) { return a[i]; }
 template <> __device__ __forceinline__ double bval<double>(const float*, const double* b, int64_t i) { return b[i]; }
@@ -1369,6 +1394,249 @@ __global__ __launch_bounds__(256) void k_apply_batched(DevTables tb, BatchVals b
     }
   }
   if (on) y[(bf + c) * K + k] = acc;
+}
+
+// The same with the rows in LDS, to the same bits: a workgroup per proton row; a
+// wave's lanes are H groups of KP = 64/H vectors.  The row's jumps are staged H*G
+// at a time per class, G jumps for each group -- source rows [h][column][K][G],
+// coefficients [h][operator][K][G] --, so that a neutron entry is the same for
+// every lane and costs two LDS reads of 4*G bytes for G products a lane.  Each
+// wave walks the entries of its run of columns, 64 of them in one load and handed
+// on by v_readlane; a column's sums over the jumps are added to the row under way
+// (in LDS) in the jumps' order.  The next batch's rows and coefficients are
+// fetched into registers while this one is worked on.  (Products and sums are
+// rounded apart, as above.)  One wave per state reads a source value and a
+// coefficient from L1 / L2 for every product and waits for each; here, FP32, one
+// pass of 64 Hamiltonians on sd 4p4n 522 -> 252 us, 32 on sd 6p6n 2.09 -> 0.57 ms,
+// 10 on pf 3p3n 3.13 -> 0.55 ms (PP and NN 107 of the 252: values read once for 4
+// columns; staging 70, the rest the entries' ten vector instructions and two LDS
+// reads).  LDS atomics in place of the read, add and write of a column's end: 398.
+template <typename T, int H, int G, int VE>
+__global__ __launch_bounds__(1024, 4) void k_apply_lanes(DevTables tb, BatchVals bv, LaneTables lt,
+                                                         const T* __restrict__ x, T* __restrict__ y) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int KP = 64 / H, J = H * G;
+  constexpr int PF = 24 / (VE * G * (int)sizeof(T) / 4), PW = 2;  // registers for the next batch
+  const int K = bv.K, LK = tb.lmax * K, wmax = tb.wcols - 1;
+  const LaneLds o(H, G, (int)sizeof(T), LK, wmax * K, lt.jumps, tb.ndelta);
+  uint2* js = reinterpret_cast<uint2*>(smem);                     // the row's jumps
+  LaneClass* cls = reinterpret_cast<LaneClass*>(smem + o.cls);
+  T* xs = reinterpret_cast<T*>(smem + o.xs);                      // [H][lmax][K][G]
+  T* yl = reinterpret_cast<T*>(smem + o.yl);                      // [lmax][K]
+  float* wb = reinterpret_cast<float*>(smem + o.wb);              // [H][operators][K][G]
+  const int tid = threadIdx.x, lane = tid & 63, NW = blockDim.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane / KP, k = min(lane % KP, K - 1);
+  const int f = blockIdx.x;
+  const int sp = tb.psec[f];
+  const int cn = tb.pconj[sp];
+  const int L = tb.nlen[cn];
+  const int vs = bv.vs, vk = bv.vk ? k : 0;
+  const int64_t bf = tb.pstart[f];
+  const int nd = tb.ndelta, nd1 = nd + 1;
+  const int jb = tb.pcls[(int64_t)f * nd1], je = tb.pcls[(int64_t)f * nd1 + nd];
+  for (int i = tid; i < nd; i += blockDim.x) {
+    LaneClass c;
+    c.p0 = tb.pcls[(int64_t)f * nd1 + i];
+    c.p1 = tb.pcls[(int64_t)f * nd1 + i + 1];
+    c.ws = tb.wstride[i];
+    c.woff = tb.woff[i];
+    const int ss = c.p0 < c.p1 ? tb.srcsec[sp * nd + i] : sp;
+    c.n = tb.nlen[tb.pconj[ss]] * K;
+    c.lp = lt.base[(int64_t)cn * nd + tb.negk[i]];
+    cls[i] = c;
+  }
+  for (int i = tid; i < je - jb; i += blockDim.x)
+    js[i] = make_uint2((uint32_t)tb.pstart[tb.p1_src[jb + i]], tb.p1_meta[jb + i]);
+  for (int i = tid; i < L * K; i += blockDim.x) xs[i] = x[bf * K + i];
+  __syncthreads();
+
+  // SPE, PP and NN: C columns of a group share a PP value
+  {
+    constexpr int C = 4;
+    const int nf0 = tb.nfirst[cn];
+    const int per = (L + NW * H - 1) / (NW * H), ca = (w * H + h) * per, cb = min(L, ca + per);
+    const int64_t e0 = tb.pp_ptr[f], e1 = tb.pp_ptr[f + 1];
+    const int E = tb.nn_emax[cn];
+    for (int c0 = 0; c0 < per; c0 += C) {
+      T acc[C];
+      int cc[C];
+#pragma unroll
+      for (int u = 0; u < C; u++) acc[u] = T(0), cc[u] = min(ca + c0 + u, L - 1);
+      if (tb.call_spe)
+#pragma unroll
+        for (int u = 0; u < C; u++)
+          acc[u] = ((T)bv.pspe[(int64_t)f * vs + vk] + (T)bv.nspe[(int64_t)(nf0 + cc[u]) * vs + vk]) * xs[cc[u] * K + k];
+      for (int64_t eb = e0; eb < e1; eb += 64) {
+        const int src = (int)tb.pstart[tb.pp_src[min(eb + lane, e1 - 1)]];
+        const int m = (int)min((int64_t)64, e1 - eb);
+#pragma unroll 4
+        for (int i = 0; i < m; i++) {
+          const int64_t r = (uint32_t)__builtin_amdgcn_readlane(src, i);
+          const T v = bval<T>(bv.pp32, bv.pp64, (eb + i) * vs + vk);
+#pragma unroll
+          for (int u = 0; u < C; u++) acc[u] += v * x[(r + cc[u]) * K + k];
+        }
+      }
+      const int64_t base = tb.nn_base[cn];
+#pragma unroll 2
+      for (int e = 0; e < E; e++) {
+        const int64_t o = base + (int64_t)e * L;
+#pragma unroll
+        for (int u = 0; u < C; u++)
+          acc[u] += bval<T>(bv.nn32, bv.nn64, (o + cc[u]) * vs + vk) * xs[tb.nn_src[o + cc[u]] * K + k];
+      }
+#pragma unroll
+      for (int u = 0; u < C; u++)
+        if (ca + c0 + u < cb) yl[cc[u] * K + k] = acc[u];
+    }
+  }
+
+  // PN.  Staging: wave w fetches for group w % H
+  const int hs = w % H, sr = (w / H) * 64 + lane, step = (NW / H) * 64;
+  const int per = (L + NW - 1) / NW, ca = min(L, w * per), cb = min(L, ca + per);  // this wave's columns
+  int cl = -1, b0 = 0, p1 = 0;
+  LaneClass c;
+  VecG<T, VE> xr[PF][G];
+  float wr[PW][G];
+  const T* xb[G];
+  const float* Wb[G];
+  uint32_t sg[G];
+  uint2 en = make_uint2(0, 0);
+  int q0 = 0, q1 = 0;
+  auto fetch = [&]() {  // the batch (cl, b0), its first part into registers
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const int j = b0 + hs * G + g;
+      const uint2 r = js[min(j, p1 - 1) - jb];
+      xb[g] = x + (int64_t)r.x * K;
+      Wb[g] = bv.W + ((int64_t)c.woff + (int64_t)(r.y & 0xff) * c.ws) * vs;
+      sg[g] = (r.y >> 8) ? 0x80000000u : 0u;
+    }
+#pragma unroll
+    for (int p = 0; p < PF; p++) {
+      const int i = (p * step + sr) * VE;
+      if (i < c.n)
+#pragma unroll
+        for (int g = 0; g < G; g++) xr[p][g] = *reinterpret_cast<const VecG<T, VE>*>(xb[g] + i);
+    }
+#pragma unroll
+    for (int p = 0; p < PW; p++) {
+      const int i = p * step + sr;
+      if (i < c.ws * K)
+#pragma unroll
+        for (int g = 0; g < G; g++) wr[p][g] = Wb[g][bv.vk ? i : i / K];
+    }
+  };
+  auto put = [&](int i, const VecG<T, VE> (&r)[G]) {
+    VecG<T, VE * G> v;
+#pragma unroll
+    for (int u = 0; u < VE; u++)
+#pragma unroll
+      for (int g = 0; g < G; g++) v.v[u * G + g] = r[g].v[u];
+    *reinterpret_cast<VecG<T, VE * G>*>(xs + ((size_t)hs * LK + i) * G) = v;
+  };
+  auto putw = [&](int i, const float (&r)[G]) {
+    VecG<float, G> v;
+#pragma unroll
+    for (int g = 0; g < G; g++) v.v[g] = __uint_as_float(__float_as_uint(r[g]) ^ sg[g]);
+    *reinterpret_cast<VecG<float, G>*>(wb + ((size_t)hs * wmax * K + i) * G) = v;
+  };
+  auto next = [&]() {
+    b0 += J;
+    bool fresh = false;
+    while (b0 >= p1) {
+      if (++cl >= nd) return false;
+      b0 = __builtin_amdgcn_readfirstlane(cls[cl].p0);
+      p1 = __builtin_amdgcn_readfirstlane(cls[cl].p1);
+      fresh = true;
+    }
+    if (fresh) {
+      c.n = __builtin_amdgcn_readfirstlane(cls[cl].n);
+      c.ws = __builtin_amdgcn_readfirstlane(cls[cl].ws);
+      c.woff = __builtin_amdgcn_readfirstlane(cls[cl].woff);
+      c.lp = __builtin_amdgcn_readfirstlane(cls[cl].lp);
+      q0 = __builtin_amdgcn_readfirstlane(lt.ptr[c.lp + ca]);
+      q1 = __builtin_amdgcn_readfirstlane(lt.ptr[c.lp + cb]);
+      if (q0 < q1) en = lt.ent[min(q0 + lane, q1 - 1)];
+    }
+    fetch();
+    return true;
+  };
+  const unsigned char* xl = reinterpret_cast<const unsigned char*>(xs + ((size_t)h * LK + k) * G);
+  const unsigned char* wl = reinterpret_cast<const unsigned char*>(wb + ((size_t)h * wmax * K + k) * G);
+  T* yk = yl + k;
+  bool more = next();
+  while (more) {
+    __syncthreads();  // the batch before is done with
+#pragma unroll
+    for (int p = 0; p < PF; p++) {
+      const int i = (p * step + sr) * VE;
+      if (i < c.n) put(i, xr[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < PW; p++) {
+      const int i = p * step + sr;
+      if (i < c.ws * K) putw(i, wr[p]);
+    }
+    for (int i = (PF * step + sr) * VE; i < c.n; i += step * VE) {
+      VecG<T, VE> r[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) r[g] = *reinterpret_cast<const VecG<T, VE>*>(xb[g] + i);
+      put(i, r);
+    }
+    for (int i = PW * step + sr; i < c.ws * K; i += step) {
+      float r[G];
+#pragma unroll
+      for (int g = 0; g < G; g++) r[g] = Wb[g][bv.vk ? i : i / K];
+      putw(i, r);
+    }
+    __syncthreads();
+    const int qa = q0, qb = q1, nj = p1 - b0;  // (jumps past the class's last are not added)
+    uint2 e = en;
+    more = next();
+    T a[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) a[g] = T(0);
+    for (int q = qa; q < qb; q += 64) {
+      if (q != qa) e = lt.ent[min(q + lane, qb - 1)];
+      // byte offsets of source and coefficient; the negative entries, the last of a column
+      const int xo = (int)(e.x & 0xffffu) * (K * G * (int)sizeof(T));
+      const int wo = (int)((e.x >> 16) & 0xffu) * (K * G * 4);
+      const int m = min(64, qb - q);
+      const uint64_t neg = __builtin_amdgcn_ballot_w64((int)e.x < 0);
+      const uint64_t last = __builtin_amdgcn_ballot_w64(lane < m && (int)e.y < 0);
+      for (int i = 0; i < m; i += 4) {
+        VecG<T, G> xv[4];
+        VecG<float, G> wv[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {  // (entries past the last come after the end of its column)
+          xv[u] = *reinterpret_cast<const VecG<T, G>*>(xl + __builtin_amdgcn_readlane(xo, i + u));
+          wv[u] = *reinterpret_cast<const VecG<float, G>*>(wl + __builtin_amdgcn_readlane(wo, i + u));
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+#pragma unroll
+          for (int g = 0; g < G; g++)
+            a[g] += (T)__uint_as_float(__float_as_uint(wv[u].v[g]) ^ ((uint32_t)(neg >> (i + u)) << 31)) * xv[u].v[g];
+          if (last >> (i + u) & 1) {  // (a group's spare lanes repeat its last vector, value and address)
+            T* p = yk + (__builtin_amdgcn_readlane((int)e.y, i + u) & 0xffff) * K;
+            T s = *p;
+#pragma unroll
+            for (int q2 = 0; q2 < H; q2++)
+#pragma unroll
+              for (int g = 0; g < G; g++)
+                if (q2 * G + g < nj) s += H == 1 ? a[g] : __shfl(a[g], q2 * KP + lane % KP, 64);
+            *p = s;
+#pragma unroll
+            for (int g = 0; g < G; g++) a[g] = T(0);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < L * K; i += blockDim.x) y[bf * K + i] = yl[i];
 }
 
 // Row kernel: y = H x with every gather from global memory and no LDS, one
@@ -2513,6 +2781,9 @@ struct bs_system {
   DevBuf<uint32_t> n1_pk, n1_pkv[3][2];
   DevBuf<uint8_t> n1_chunk;
   DevBuf<uint32_t> n1_pkr;
+  DevBuf<int32_t> lane_base, lane_ptr;  // k_apply_lanes
+  DevBuf<uint2> lane_ent;
+  int lane_jumps = 0;  // most jumps of a row
   DevBuf<float> pspe_sd, nspe_sd, pp_val32, nn_val32, W;
   DevBuf<double> pp_val64, nn_val64;
   bsl::Owner like;              // tables of the separate PP and NN kernels
@@ -2871,6 +3142,30 @@ void upload_tables(bs_system* s) {
   s->n1_emax.upload(n1_emax);
   s->n1_pk.upload(n1_pk);
   s->n1_chunk.upload(n1_chunk);
+  {
+    // the same entries column by column, for waves that walk a column
+    std::vector<int32_t> base((size_t)N.nsec * nd), ptr;
+    std::vector<uint2> ent;
+    for (int c = 0; c < N.nsec; c++)
+      for (int k = 0; k < nd; k++) {
+        base[(size_t)c * nd + k] = (int32_t)ptr.size();
+        const uint32_t pad = (uint32_t)t.class_size[k] << 16;
+        for (int col = 0; col < nlen[c]; col++) {
+          ptr.push_back((int32_t)ent.size());
+          for (int e = 0; e < n1_emax[(size_t)c * nd + k]; e++) {
+            const uint32_t pk = n1_pk[n1_base[(size_t)c * nd + k] + (int64_t)e * nlen[c] + col];
+            if (pk == pad) continue;
+            ent.push_back(make_uint2((pk & 0xffffffu) | ((pk >> 24 & 1u) << 31), (uint32_t)col));
+          }
+          if ((int32_t)ent.size() > ptr.back()) ent.back().y |= 1u << 31;
+        }
+        ptr.push_back((int32_t)ent.size());
+      }
+    for (int f = 0; f < nP; f++) s->lane_jumps = std::max(s->lane_jumps, pcls[(size_t)f * (nd + 1) + nd] - pcls[(size_t)f * (nd + 1)]);
+    s->lane_base.upload(base);
+    s->lane_ptr.upload(ptr);
+    s->lane_ent.upload(ent);
+  }
   {
     std::vector<uint32_t> v(n1_pk.size());
     for (size_t i = 0; i < n1_pk.size(); i++) {
@@ -3910,7 +4205,7 @@ constexpr int kMaxBatch = 64;
 
 int batch_blocks(int64_t D) { return (int)std::min<int64_t>(std::max<int64_t>((D + 63) / 64, 1), 512); }
 
-// Multi-vector kernels: variant 0 = one wave per basis state (lane = vector;
+// Multi-vector kernels: variant 0 = k_apply_lanes or one wave per state (lane = vector;
 // small bases), 1 + 2*gi + map = k_apply_multi with G = 1 << gi staged rows
 // and identity (map 0) or XCD-aware (map 1) workgroup order.
 constexpr int kNumMulti = 7;
@@ -3972,6 +4267,38 @@ bool multi_fits(const bs_system* s, int v, int K, size_t tsize, bool shared) {
   return (size_t)G * K * s->dt.lmax * tsize + (size_t)kWbRows * G * K * sizeof(float) <= kLdsLimit;
 }
 
+// k_apply_lanes where its rows fit: the most groups that K and the LDS leave, with
+// two staged jumps a group if they fit; two workgroups of 8 waves on a CU, else
+// one of 16.  false: not even one group's rows fit, k_apply_batched it is.
+template <typename T>
+bool launch_lanes(const bs_system* s, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
+  const DevTables& d = s->dt;
+  if (d.lmax > 4096 || d.dim > (int64_t)UINT32_MAX) return false;
+  auto lds = [&](int H, int G) {
+    return (size_t)LaneLds(H, G, (int)sizeof(T), d.lmax * bv.K, (d.wcols - 1) * bv.K, s->lane_jumps, d.ndelta).bytes;
+  };
+  int H = bv.K <= 8 ? 8 : bv.K <= 16 ? 4 : bv.K <= 32 ? 2 : 1;
+  while (H > 1 && lds(H, 1) > kLdsLimit) H /= 2;
+  if (lds(H, 1) > kLdsLimit) return false;
+  const int G = lds(H, 2) <= kLdsLimit ? 2 : 1;
+  const int threads = lds(H, G) <= kLdsLimit / 2 ? 512 : 1024;
+  constexpr int V = 16 / (int)sizeof(T);
+  const bool vec = bv.K % V == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  const LaneTables lt{s->lane_base.p, s->lane_ptr.p, s->lane_ent.p, s->lane_jumps};
+  auto go = [&](auto fn) {
+    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)kLdsLimit));
+    hipLaunchKernelGGL(fn, dim3(d.nP), dim3(threads), lds(H, G), st, d, bv, lt, x, y);
+    HIP_OK(hipGetLastError());
+  };
+#define BS_LANES(HH, GG) \
+  if (H == HH && G == GG) vec ? go(k_apply_lanes<T, HH, GG, V>) : go(k_apply_lanes<T, HH, GG, 1>);
+  BS_LANES(1, 1) BS_LANES(2, 1) BS_LANES(4, 1) BS_LANES(8, 1)
+  BS_LANES(1, 2) BS_LANES(2, 2) BS_LANES(4, 2) BS_LANES(8, 2)
+#undef BS_LANES
+  return true;
+}
+
 // k_apply_ktiles on the two-row tiles (map 0: sector order, 1: XCD-grouped)
 template <typename T, int K>
 void launch_ktiles(const bs_system* s, int map, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
@@ -3998,6 +4325,7 @@ void launch_batched_v(const bs_system* s, int v, const BatchVals& bv, const T* x
   const DevTables& d = s->dt;
   if (bv.K < 1 || bv.K > kMaxBatch) throw std::runtime_error("batch size must be in 1..64");
   if (v == 0) {
+    if (launch_lanes<T>(s, bv, x, y, st)) return;
     const int ny = (d.lmax + 3) / 4;
     hipLaunchKernelGGL(k_apply_batched<T>, dim3(d.nP, ny), dim3(256), 0, st, d, bv, x, y);
     HIP_OK(hipGetLastError());
