@@ -818,6 +818,202 @@ __global__ void k_normalize(T* __restrict__ v, const T* __restrict__ w, const do
     v[i] = (T)((double)w[i] * m);
 }
 
+// ---- the vector work of a Lanczos step after H v_i and <v_i, w>, in three
+// passes.  Every workgroup adds up the partial sums that the kernel before left
+// (L2 gives them in about a microsecond) instead of waiting for a kernel that
+// does only that, and an update and the dots that follow it share a pass.  On
+// small bases the step is launches of some 4 us: sd 6p6n FP64 (D = 93,710)
+// nine of them after the first dot, 45 us a step, here three.
+
+// sum of p[0 .. n), the same in every lane of every wave
+__device__ __forceinline__ double wave_total(const double* __restrict__ p, int n) {
+  double s = 0.0;
+  for (int b = threadIdx.x & 63; b < n; b += 64) s += p[b];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
+// alpha = sum of dot[0 .. nb); w -= T(alpha v); partial sums of <V_j, w>, j < m,
+// of workgroup b at part[b * sb + j * sj].  A tile of w goes through LDS to the
+// four waves, each of which has every fourth vector: 32 vectors are in flight
+// and a sum crosses one wave only.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_step_dots(T* __restrict__ w, const T* __restrict__ v,
+                                                      const double* __restrict__ dot, int nb, double* __restrict__ alpha,
+                                                      const T* __restrict__ V, int64_t ld, int m, int64_t D,
+                                                      double* __restrict__ part, int sb, int sj) {
+  using V16 = typename Vec16<T>::type;
+  constexpr int VW = Vec16<T>::n, NW = kBlock / 64, U = 8;
+  __shared__ V16 tile[kBlock];
+  const bool vec = ((((uintptr_t)V | (uintptr_t)w | (uintptr_t)v) & 15) == 0) && (ld % VW == 0);
+  const int64_t nv = vec ? D / VW : 0;
+  const int64_t chunk = (nv + gridDim.x - 1) / gridDim.x;
+  const int64_t lo = (int64_t)blockIdx.x * chunk;
+  const int64_t hi = lo + chunk < nv ? lo + chunk : nv;
+  // elements one by one: the tail, or all of them where they are not aligned
+  const int64_t s0 = nv * VW;
+  const int64_t sc = (D - s0 + gridDim.x - 1) / gridDim.x;
+  const int64_t slo = s0 + (int64_t)blockIdx.x * sc, shi = min(slo + sc, D);
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  V16* w16 = reinterpret_cast<V16*>(w);
+  const double s = wave_total(dot, nb);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *alpha = s;
+  for (int64_t i = slo + threadIdx.x; i < shi; i += kBlock) w[i] = w[i] - (T)(s * (double)v[i]);
+  for (int j0 = 0; j0 == 0 || j0 < m; j0 += NW * U) {
+    double a[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) a[u] = 0.0;
+    for (int64_t t0 = lo; t0 < hi; t0 += kBlock) {
+      const int n = (int)min((int64_t)kBlock, hi - t0);
+      if ((int)threadIdx.x < n) {
+        V16 wi = w16[t0 + threadIdx.x];
+        if (j0 == 0) {
+          const V16 vi = reinterpret_cast<const V16*>(v)[t0 + threadIdx.x];
+          T* pw = reinterpret_cast<T*>(&wi);
+          const T* pv = reinterpret_cast<const T*>(&vi);
+#pragma unroll
+          for (int e = 0; e < VW; e++) pw[e] = pw[e] - (T)(s * (double)pv[e]);
+          w16[t0 + threadIdx.x] = wi;
+        }
+        tile[threadIdx.x] = wi;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kBlock; r += 64)
+        if (r + lane < n && m > 0) {
+          const V16 wi = tile[r + lane];
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            const int j = min(j0 + u * NW + wid, m - 1);
+            a[u] += dot16(reinterpret_cast<const V16*>(V + (int64_t)j * ld)[t0 + r + lane], wi);
+          }
+        }
+      __syncthreads();
+    }
+    if (slo < shi) {  // (the same in the whole workgroup)
+      __syncthreads();
+      for (int64_t i = slo + lane; i < shi; i += 64)
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int j = j0 + u * NW + wid;
+          if (j < m) a[u] += (double)V[(int64_t)j * ld + i] * (double)w[i];
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+      for (int u = 0; u < U; u++) a[u] += __shfl_xor(a[u], o, 64);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int j = j0 + u * NW + wid;
+      if (j < m && lane == 0) part[(int64_t)blockIdx.x * sb + (int64_t)j * sj] = a[u];
+    }
+  }
+}
+
+// w -= T(sum_j d_j V_j), j < m, and norm[b] = workgroup b's share of <w, w>.
+// SUM: d_j is the sum of d[j * nb .. (j + 1) * nb), m <= kStepSums / nb
+constexpr int kStepSums = 8192;
+template <typename T, bool SUM>
+__global__ __launch_bounds__(kBlock) void k_step_axpy(T* __restrict__ w, const T* __restrict__ V, int64_t ld, int m,
+                                                      const double* __restrict__ d, int nb, int64_t D,
+                                                      double* __restrict__ norm) {
+  using V16 = typename Vec16<T>::type;
+  constexpr int VW = Vec16<T>::n;
+  extern __shared__ double dj[];
+  __shared__ double red[kBlock / 64];
+  if constexpr (SUM) {
+    constexpr int NW = kBlock / 64, U = 8;  // eight sums of a wave at a time
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    for (int j0 = wid; j0 < m; j0 += NW * U) {
+      double t[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) t[u] = 0.0;
+#pragma unroll 4
+      for (int b = lane; b < nb; b += 64)
+#pragma unroll
+        for (int u = 0; u < U; u++)
+          t[u] += d[(int64_t)min(j0 + u * NW, m - 1) * nb + b];
+      for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int u = 0; u < U; u++) t[u] += __shfl_xor(t[u], o, 64);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (j0 + u * NW < m && lane == 0) dj[j0 + u * NW] = t[u];
+    }
+    __syncthreads();
+  }
+  auto c = [&](int j) { return SUM ? dj[j] : d[j]; };
+  const bool vec = ((((uintptr_t)V | (uintptr_t)w) & 15) == 0) && (ld % VW == 0);
+  const int64_t nv = vec ? D / VW : 0;
+  V16* w16 = reinterpret_cast<V16*>(w);
+  double n2 = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+    double s[VW];
+#pragma unroll
+    for (int e = 0; e < VW; e++) s[e] = 0.0;
+#pragma unroll 8
+    for (int j = 0; j < m; j++) {
+      const V16 v = reinterpret_cast<const V16*>(V + (int64_t)j * ld)[i];
+      const T* pv = reinterpret_cast<const T*>(&v);
+#pragma unroll
+      for (int e = 0; e < VW; e++) s[e] += c(j) * (double)pv[e];
+    }
+    V16 o = w16[i];
+    T* po = reinterpret_cast<T*>(&o);
+#pragma unroll
+    for (int e = 0; e < VW; e++) po[e] = po[e] - (T)s[e];
+    w16[i] = o;
+    n2 += dot16(o, o);
+  }
+  for (int64_t i = nv * VW + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < D;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    double s = 0.0;
+    for (int j = 0; j < m; j++) s += c(j) * (double)V[(int64_t)j * ld + i];
+    const T o = w[i] - (T)s;
+    w[i] = o;
+    n2 += (double)o * (double)o;
+  }
+  for (int o = 32; o > 0; o >>= 1) n2 += __shfl_down(n2, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = n2;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int q = 0; q < kBlock / 64; q++) t += red[q];
+    norm[blockIdx.x] = t;
+  }
+}
+
+// beta_i = sqrt(sum of norm[0 .. nb)), v = T(double(w) / beta_i), zero where the
+// Krylov space is the whole space (last).  The step needs the host's decision
+// when beta_i is below 0.1 of its scale (beta_{i-1}, or |H v_i| on a cycle's
+// first step, with the arrow couplings beta[0:kst]) or not finite; the first
+// such step is kept.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_step_next(T* __restrict__ v, const T* __restrict__ w,
+                                                      const double* __restrict__ norm, int nb,
+                                                      const double* __restrict__ alpha, double* __restrict__ beta, int i,
+                                                      int kst, int* __restrict__ first, bool last, int64_t D) {
+  const double b = sqrt(wave_total(norm, nb));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    beta[i] = b;
+    if (!last) {
+      const double a = alpha[i];
+      double scale;
+      if (i == kst) {
+        double s2 = a * a + b * b;
+        for (int j = 0; j < kst; j++) s2 += beta[j] * beta[j];
+        scale = sqrt(s2);
+      } else {
+        scale = beta[i - 1];
+      }
+      if (!(b >= 0.1 * scale) || b == 0.0 || !isfinite(a) || !isfinite(b)) atomicMin(first, i);
+    }
+  }
+  const double q = 1.0 / b;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < D; e += (int64_t)gridDim.x * blockDim.x)
+    v[e] = last ? T(0) : (T)((double)w[e] * q);
+}
+
 // seeded values in [-1, 1): SplitMix64 (Steele, Lea, Flood 2014) of the index
 template <typename T>
 __global__ void k_pivot_random(T* __restrict__ v, int64_t n, uint64_t seed) {
@@ -2360,24 +2556,6 @@ __global__ void k_bloss(const double* __restrict__ dots, int m, int K, int* __re
   if (dmax <= 1e-5) flags[k] = 0;
 }
 
-// single Lanczos run: step i needs the host's decision when beta_i is below
-// 0.1 of its scale (beta_{i-1}, or |H v_i| on a cycle's first step, with the
-// arrow couplings beta[0:kst]) or not finite; the first such step is kept
-__global__ void k_bflag(const double* __restrict__ alpha, const double* __restrict__ beta, int i, int kst,
-                        int* __restrict__ first) {
-  if (threadIdx.x != 0) return;
-  const double a = alpha[i], b = beta[i];
-  double scale;
-  if (i == kst) {
-    double s2 = a * a + b * b;
-    for (int j = 0; j < kst; j++) s2 += beta[j] * beta[j];
-    scale = sqrt(s2);
-  } else {
-    scale = beta[i - 1];
-  }
-  if (!(b >= 0.1 * scale) || b == 0.0 || !isfinite(a) || !isfinite(b)) atomicMin(first, i);
-}
-
 // w -= T(sum_j d_j V_j) and then w /= norm, for members with flags >= minflag
 template <typename T>
 __global__ void k_bmultiaxpy_m(T* __restrict__ w, const T* __restrict__ V, int64_t ldv, int m,
@@ -3463,6 +3641,8 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
   HIP_OK(hipDeviceSynchronize());
   const int mtot = niter + 1;
   const int nb = grid_for(D) < 1024 ? grid_for(D) : 1024;
+  // workgroups of a step's passes: a 16-byte word a thread
+  const int nbs = (int)std::min<int64_t>(nb, (D + kBlock * Vec16<T>::n - 1) / (kBlock * Vec16<T>::n));
   // Lanczos vectors at a stride of whole 64-element blocks: every v_i starts
   // 256-byte aligned, so the streaming passes use 16-byte loads
   const int64_t ld = (D + 63) / 64 * 64;
@@ -3570,7 +3750,7 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
     return p->conv_test == 3 ? mx : std::sqrt(s2) / ncheck;
   };
   // A step needs no host round trip: v_{i+1} = w / beta_i at once, and
-  // k_bflag records on the device the first step whose beta falls below 0.1
+  // k_step_next records on the device the first step whose beta falls below 0.1
   // of its scale (or is not finite).  Each time the host reads alpha/beta
   // anyway (a convergence check, a restart, the end) it first reads that
   // step; if there is one, the steps after it are discarded and it is redone
@@ -3586,16 +3766,6 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
     k_multidot<T><<<nb, kBlock, 0, st>>>(v, D, 1, v, D, part.p);
     k_reduce<<<1, kBlock, 0, st>>>(part.p, nb, 1, dots.p + m, 1);
     k_normalize<T><<<g, kBlock, 0, st>>>(v, v, dots.p + m, D);
-  };
-  auto next_vector = [&](int i, int kst) {
-    T* vn = V.p + (int64_t)(i + 1) * ld;
-    if (i + 1 >= D) {
-      k_fill<T><<<g, kBlock, 0, st>>>(vn, T(0), D);
-      return;
-    }
-    // the arrow couplings of a thick restart sit in beta[0:kst]
-    k_bflag<<<1, 64, 0, st>>>(d_alpha, d_beta, i, kst, d_first);
-    k_normalize<T><<<g, kBlock, 0, st>>>(vn, w.p, d_beta + i, D);
   };
   auto next_vector_host = [&](int i, int kst) {
     T* vn = V.p + (int64_t)(i + 1) * ld;
@@ -3625,7 +3795,7 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
       random_restarts++;
       return;
     }
-    // v_{i+1} = w_i / beta_i is already in place (next_vector ran first; w
+    // v_{i+1} = w_i / beta_i is already in place (k_step_next ran first; w
     // itself has been overwritten by the later steps since)
     if (bi < 0.1 * scale) {
       const int m = i + 1;
@@ -3671,17 +3841,21 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
     T* vi = V.p + (int64_t)i * ld;
     launch_apply<T>(s, vi, w.p, 0, st);
     total_mv++;
-    k_multidot<T><<<nb, kBlock, 0, st>>>(vi, D, 1, w.p, D, part.p);
-    k_reduce<<<1, kBlock, 0, st>>>(part.p, nb, 1, d_alpha + i, 0);
-    k_sub_scaled<T><<<g, kBlock, 0, st>>>(w.p, vi, d_alpha + i, D);
-    if (i > 0) {
-      k_multidot<T><<<nb, kBlock, 0, st>>>(V.p, ld, i, w.p, D, part.p);
-      k_reduce<<<i, kBlock, 0, st>>>(part.p, nb, i, dots.p, 0);
-      k_multiaxpy<T><<<g, kBlock, 0, st>>>(w.p, V.p, ld, i, dots.p, D);
+    // the last nbs of part: <v_i, w>, then <w, w>; the first: the dots with V
+    double* dot = part.p + (size_t)nbs * (mtot - 1);
+    k_multidot<T><<<nbs, kBlock, 0, st>>>(vi, D, 1, w.p, D, dot);
+    // in each workgroup of the next kernel at most kStepSums partial sums; on
+    // large bases with many vectors (nbs = 1,024: from 9) one more launch costs less
+    const bool sum = (int64_t)nbs * i <= kStepSums;
+    k_step_dots<T><<<nbs, kBlock, 0, st>>>(w.p, vi, dot, nbs, d_alpha + i, V.p, ld, i, D, part.p, sum ? 1 : i, sum ? nbs : 1);
+    if (sum) {
+      k_step_axpy<T, true><<<nbs, kBlock, sizeof(double) * i, st>>>(w.p, V.p, ld, i, part.p, nbs, D, dot);
+    } else {
+      k_reduce<<<i, kBlock, 0, st>>>(part.p, nbs, i, dots.p, 0);
+      k_step_axpy<T, false><<<nbs, kBlock, 0, st>>>(w.p, V.p, ld, i, dots.p, nbs, D, dot);
     }
-    k_multidot<T><<<nb, kBlock, 0, st>>>(w.p, D, 1, w.p, D, part.p);
-    k_reduce<<<1, kBlock, 0, st>>>(part.p, nb, 1, d_beta + i, 1);
-    next_vector(i, kstart);
+    k_step_next<T><<<g, kBlock, 0, st>>>(V.p + (int64_t)(i + 1) * ld, w.p, dot, nbs, d_alpha, d_beta, i, kstart, d_first,
+                                         i + 1 >= D, D);
     HIP_OK(hipGetLastError());
   };
   // Ritz pairs of the projected matrix on v_0 .. v_{m-1}: the locked Ritz
