@@ -17,7 +17,7 @@ HIP_FLAGS = [
 ]
 
 
-SOURCES = ("bs_engine.hip", "bs_like.hip", "bs_tables.cpp")
+SOURCES = ("bs_engine.hip", "bs_like.hip", "bs_short.hip", "bs_tables.cpp")
 
 
 def build_native(verbose=False):

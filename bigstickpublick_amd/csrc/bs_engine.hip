@@ -35,6 +35,7 @@
 #include "../../include/bigstick_amd.h"
 #include "bs_tables.hpp"
 #include "bs_like.hpp"
+#include "bs_short.hpp"
 #include <rocsolver/rocsolver.h>
 #include <atomic>
 #include <mutex>
@@ -2965,6 +2966,7 @@ struct bs_system {
   DevBuf<float> pspe_sd, nspe_sd, pp_val32, nn_val32, W;
   DevBuf<double> pp_val64, nn_val64;
   bsl::Owner like;              // tables of the separate PP and NN kernels
+  bss::Owner brief;             // tables of the short-row kernel
 };
 
 namespace {
@@ -3191,8 +3193,10 @@ void upload_tables(bs_system* s) {
     if (P.start[f] < 0 || P.start[f] + nlen[P.conj[P.sdsec[f]]] > t.dim) throw std::runtime_error("row outside the vector");
   // tiles for each R, and two workgroup->tile maps: identity (sector order)
   // and XCD-grouped (below)
+  std::vector<int32_t> tile_f0[3], tile_nr[3];
+  std::vector<int64_t> tpp_ptr[3];
   for (int v = 0; v < 3; v++) {
-    std::vector<int32_t> f0, nr;
+    std::vector<int32_t>&f0 = tile_f0[v], &nr = tile_nr[v];
     for (int sp = 0; sp < P.nsec; sp++)
       for (int64_t f = P.secfirst[sp]; f < P.secfirst[sp] + P.seccount[sp]; f += kTileRows[v]) {
         f0.push_back((int32_t)f);
@@ -3206,7 +3210,8 @@ void upload_tables(bs_system* s) {
       // PP source union per tile (sources of all R rows, each listed once)
       const int R = kTileRows[v];
       const bs::TwoBody& T = t.tb[0];
-      std::vector<int64_t> ptr(nt + 1, 0);
+      std::vector<int64_t>& ptr = tpp_ptr[v];
+      ptr.assign(nt + 1, 0);
       std::vector<uint32_t> src;
       std::vector<float> v32;
       std::vector<double> v64;
@@ -3440,6 +3445,9 @@ void upload_tables(bs_system* s) {
   d.wstride = s->wstride.p;
   d.negk = s->negk.p;
   if (s->tiles_ok) bsl::build(s->like, t, s->pstart.p, s->psec.p, s->pconj.p, s->nlen.p, nlen, s->pp_ptr.p, s->pp_src.p, s->pp_val64.p);
+  if (s->tiles_ok)
+    bss::build(s->brief, {t, nlen, srcsec, pcls, p1_src, p1_meta, n1q_base, n1_chunk, nn_base, nn_emax, woff, wstride, negk,
+                          tile_f0, tile_nr, tpp_ptr});
   s->uploaded = true;
 }
 
@@ -3503,15 +3511,19 @@ void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumu
 // pf 6p6n 21.0 -> 18.9 ms, FP64 42.7 -> 35.2 ms); on short rows the two extra
 // launches and the tiles' padding cost more (pf 2p3n 32 -> 68 us).
 constexpr int kLikeVariant = kNumVariants;
-constexpr int kRowsVariant = kLikeVariant + kNumShapes;
+// After them the short-row kernel's shapes (bs_short.hip)
+constexpr int kShortVariant = kLikeVariant + kNumShapes;
+constexpr int kRowsVariant = kShortVariant + bss::kShapes;
 constexpr int kAllVariants = kRowsVariant + 1;
 constexpr int64_t kLikeDim = 1000000;  // basis size from which they are the default
-constexpr bool is_like(int v) { return v >= kLikeVariant && v < kRowsVariant; }
+constexpr bool is_like(int v) { return v >= kLikeVariant && v < kShortVariant; }
+constexpr bool is_short(int v) { return v >= kShortVariant && v < kRowsVariant; }
 
 template <typename T>
 size_t lds_bytes(const bs_system* s, int v) {
   if (v == kRowsVariant) return 0;
   if (!s->tiles_ok) return SIZE_MAX;
+  if (is_short(v)) return s->brief.has(v - kShortVariant, sizeof(T) == 4) ? 0 : SIZE_MAX;
   if (is_like(v) && !s->like.ok) return SIZE_MAX;
   return lds_bytes_rg<T>(s, kVarR[v % kNumShapes], kVarG[v % kNumShapes]);
 }
@@ -3537,6 +3549,24 @@ void launch_cpt(bs_system* s, int v, const T* x, T* y, int accumulate, hipStream
 }
 
 template <typename T>
+void launch_short(bs_system* s, int shape, const T* x, T* y, int accumulate, hipStream_t st) {
+  const int ri = bss::kRows[shape] == 1 ? 0 : (bss::kRows[shape] == 2 ? 1 : 2);
+  bss::Tab z{};
+  z.call_spe = s->dt.call_spe;
+  z.quad = s->n1_pkv[shape >= bss::kSplit ? 1 : ri][sizeof(T) == 4 ? 0 : 1].p;
+  z.W = s->W.p;
+  z.pp_src = s->tpp_src[ri].p;
+  z.pp32 = s->tpp_val32[ri].p;
+  z.pp64 = s->tpp_val64[ri].p;
+  z.nn_src = s->nn_src.p;
+  z.nn32 = s->nn_val32.p;
+  z.nn64 = s->nn_val64.p;
+  z.pspe = s->pspe_sd.p;
+  z.nspe = s->nspe_sd.p;
+  bss::apply(s->brief, shape, z, x, y, accumulate, st);
+}
+
+template <typename T>
 void launch_apply_v(bs_system* s, int v, const T* x, T* y, int accumulate, hipStream_t st) {
   if (v < 0 || v >= kAllVariants) throw std::runtime_error("bad kernel variant");
   if (lds_bytes<T>(s, v) > kLdsLimit) throw std::runtime_error("kernel variant does not fit in LDS");
@@ -3545,6 +3575,10 @@ void launch_apply_v(bs_system* s, int v, const T* x, T* y, int accumulate, hipSt
       hipLaunchKernelGGL(k_apply_rows<T>, dim3(s->nrows_wg), dim3(256), 0, st, s->dt, s->rows_f.p, s->rows_c.p, x, y,
                          accumulate);
     HIP_OK(hipGetLastError());
+    return;
+  }
+  if (is_short(v)) {
+    launch_short<T>(s, v - kShortVariant, x, y, accumulate, st);
     return;
   }
   switch (s->cpt) {
@@ -3573,6 +3607,9 @@ int autotune(bs_system* s, hipStream_t st) {
   int bestv = -1;
   for (int v = 0; v < kAllVariants; v++) {
     if (lds_bytes<T>(s, v) > kLdsLimit) continue;
+    // on short rows no other kernel came near the short-row one's shapes
+    // (bs_short.hip: two to four times slower in every case)
+    if (!is_short(v) && s->brief.usual(sizeof(T) == 4) >= 0) continue;
     // on large bases the staged-after tiles never won against the PF ones
     // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
     if (v < 2 * kNumShapes && s->like.ok && D >= kLikeDim) continue;
@@ -3597,9 +3634,10 @@ template <typename T>
 void launch_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st) {
   const int di = sizeof(T) == 4 ? 0 : 1;
   if (s->variant[di] < 0) {
-    // until autotuned: the largest tile that fits, on large bases with the
-    // separate PP and NN kernels
-    int v = s->like.ok && s->t.dim >= kLikeDim ? kRowsVariant - 1 : 2 * kNumShapes - 1;
+    // until autotuned: on short rows a shape of their kernel; else the largest
+    // tile that fits, on large bases with the separate PP and NN kernels
+    const int sh = s->brief.usual(sizeof(T) == 4);
+    int v = sh >= 0 ? kShortVariant + sh : s->like.ok && s->t.dim >= kLikeDim ? kShortVariant - 1 : 2 * kNumShapes - 1;
     while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
     s->variant[di] = v >= 0 ? v : kRowsVariant;
   }
@@ -5546,6 +5584,16 @@ int bs_variant_info(int v, int* rows, int* staged, int* xcd_map, int* prefetch) 
     if (staged) *staged = 0;
     if (xcd_map) *xcd_map = 0;
     if (prefetch) *prefetch = 0;
+    return 0;
+  }
+  if (is_short(v)) {
+    // every row of the tile staged, in workgroups of 8 or 16 waves; 4: one row, two
+    // jumps, a column's sum in order
+    const int sh = v - kShortVariant;
+    if (rows) *rows = bss::kRows[sh];
+    if (staged) *staged = sh < bss::kSplit ? bss::kRows[sh] : 2;
+    if (xcd_map) *xcd_map = bss::kWaves[sh] == 16;
+    if (prefetch) *prefetch = sh < bss::kSplit ? 3 : 4;
     return 0;
   }
   if (rows) *rows = kVarR[v % kNumShapes];
