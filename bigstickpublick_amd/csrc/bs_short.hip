@@ -8,11 +8,15 @@
 // wave walks its share of the batches, of the PP sources and of the NN slots for
 // one 64-column chunk, and the shares are added up in LDS at the end.
 //
-// Tiles / here, us: sd 4p4n FP64 36.6 / 13.2, sd 5p6n FP64
-// 71 / 26, sd 6p6n FP64 80 / 30, pf 3p3n FP32 88 / 33, pf 4p3n FP32 296 / 118, pf
-// 8p3n FP32 9829 / 5549, pf 8p2n FP32 6847 (rows) / 1832.  On small bases the launch
-// (some 5 us) and the chain tile - batch - source rows - walk - sum bound it, on
-// large ones the LDS reads of the walk, with lanes idle past a row's end.
+// Tiles / here, us: sd 4p4n FP64 36.6 / 13.2, sd 5p6n FP64 71 / 26, sd 6p6n FP64 80 / 30,
+// pf 3p3n FP32 88 / 33, pf 4p3n FP32 296 / 118, pf 8p3n FP32 9829 / 5549, pf 8p2n FP32
+// 6847 (rows) / 1832.  From some hundred columns on PP and NN go to their own kernels
+// (bs_like.hip): pf 4p4n FP32 460 / 319 (404 with PP and NN here), FP64 700 / 552, pf 6p4n
+// FP32 4037 / 3011.  Columns cut into equal runs over the waves, so that nine chunks
+// load 16 waves evenly, gained nothing (pf 6p4n 3037, pf 4p3n FP64 168 -> 207).  On
+// small bases the launch (some 5 us) and the chain tile - batch - source rows - walk -
+// sum bound it, on large ones the LDS reads of the walk, with lanes idle past a row's
+// end.
 #include "bs_short.hpp"
 
 #include <algorithm>
@@ -48,12 +52,14 @@ template <> __device__ __forceinline__ const double* pick<double>(const float*, 
 // 64-column chunks of the longest row.  LDS: the tile's own rows [column][R], then
 // per batch the source rows [column][R] and the signed coefficients [2 * operator +
 // sign][R] (the entry quads hold byte offsets into both).
-template <typename T, int R, int NW, int CH>
-__global__ __launch_bounds__(NW * 64) void k_short(Tab z, int S, const T* __restrict__ x, T* __restrict__ y, int accumulate) {
+// (CH 9: launched with waves enough for every chunk, more than 8.)
+template <typename T, int R, int WAVES, int CH>
+__global__ __launch_bounds__((CH == 9 && WAVES < 10 ? 10 : WAVES) * 64) void k_short(Tab z, int S, const T* __restrict__ x, T* __restrict__ y, int accumulate) {
   extern __shared__ __align__(16) unsigned char smem[];
   using XV = Row<T, R>;
   using WV = Row<float, R>;
-  constexpr int BS = 4 + 2 * R;  // words of a batch
+  constexpr int BS = 6 + 2 * R;  // words of a batch
+  const int NW = CH == 9 ? (int)blockDim.x >> 6 : WAVES;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // workgroup b runs on XCD b % 8: on bases of many tiles, runs of 32 tiles, which
   // share source rows, each
@@ -71,7 +77,7 @@ __global__ __launch_bounds__(NW * 64) void k_short(Tab z, int S, const T* __rest
   T acc[R];
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = T(0);
-  for (int c = tid; c < L; c += NW * 64) {
+  for (int c = tid; z.like && c < L; c += NW * 64) {
     XV v;
 #pragma unroll
     for (int r = 0; r < R; r++) v.v[r] = r < nr ? x[base + (uint32_t)(r * L + c)] : T(0);
@@ -88,7 +94,7 @@ __global__ __launch_bounds__(NW * 64) void k_short(Tab z, int S, const T* __rest
       unsigned char* at = area + (uint32_t)(i - p0) * bbytes;
       uint32_t src[R], wr[R];
 #pragma unroll
-      for (int r = 0; r < R; r++) src[r] = rec[4 + 2 * r], wr[r] = rec[5 + 2 * r];
+      for (int r = 0; r < R; r++) src[r] = rec[6 + 2 * r], wr[r] = rec[7 + 2 * r];
       XV v[CH];
       WV c[2];
 #pragma unroll
@@ -113,7 +119,7 @@ __global__ __launch_bounds__(NW * 64) void k_short(Tab z, int S, const T* __rest
         if (lane + 64 * u < 2 * (ws + 1)) reinterpret_cast<WV*>(at + xbytes)[lane + 64 * u] = c[u];
     }
     __syncthreads();
-    if (p0 == b0) {
+    if (p0 == b0 && z.like) {
       if (z.call_spe && sub == 0) {
         const XV v = own[cl];
 #pragma unroll
@@ -178,7 +184,7 @@ __global__ __launch_bounds__(NW * 64) void k_short(Tab z, int S, const T* __rest
       if (lane < m) {
         const uint32_t* rec = z.batch + (size_t)(p0 + sub + lane * nsub) * BS;
         dq = rec[0];
-        dE = rec[2] >> (8 * chunk) & 255u;
+        dE = rec[2 + (chunk >> 2)] >> (8 * (chunk & 3)) & 255u;
       }
       const u4* quad = reinterpret_cast<const u4*>(z.quad);
       u4 nx[3] = {};
@@ -293,7 +299,7 @@ __global__ __launch_bounds__(NW * 64) void k_chain(Tab z, const float* __restric
   const int m = walks ? max((nb - sub + nsub - 1) / nsub, 0) : 0;  // (64 at most)
   uint32_t dq = 0, dE = 0;
   if (lane < m) {
-    const uint32_t* rec = z.pair + (size_t)(b0 + sub + lane * nsub) * 8;
+    const uint32_t* rec = z.pair + (size_t)(b0 + sub + lane * nsub) * 10;
     dq = rec[0];
     dE = rec[2] >> (8 * chunk) & 255u;
   }
@@ -309,9 +315,9 @@ __global__ __launch_bounds__(NW * 64) void k_chain(Tab z, const float* __restric
   if (m > 0) entries(0);
   for (int c = tid; c < L; c += NW * 64) own[c] = x[base + (uint32_t)c];
   for (int b = w; b < nb; b += NW) {
-    const cptr<uint32_t> rec = cst(z.pair) + (size_t)(b0 + b) * 8;
+    const cptr<uint32_t> rec = cst(z.pair) + (size_t)(b0 + b) * 10;
     const int Li = rec[1] & 0xffff, ws = rec[1] >> 16;
-    const uint32_t s0 = rec[4], w0 = rec[5], s1 = rec[6], w1 = rec[7];
+    const uint32_t s0 = rec[6], w0 = rec[7], s1 = rec[8], w1 = rec[9];
     unsigned char* at = area + (uint32_t)b * bbytes;
     V2 v[4], c[2];
 #pragma unroll
@@ -420,15 +426,16 @@ constexpr size_t kManyJumps = (size_t)1 << 20, kMaxJumps = (size_t)1 << 25;
 template <typename T, int SH, int CH>
 void launch(const Owner& o, const Tab& z, const T* x, T* y, int accumulate, hipStream_t st) {
   constexpr int R = kRows[SH], NW = kWaves[SH];
+  const int ncmax = (o.lmax + 63) / 64, waves = CH < 9 ? NW : NW == 8 ? ncmax : std::min(16, 2 * ncmax);
   const Owner::Set& q = o.set[set_of(R)];
   const size_t own = (size_t)o.ls * R * sizeof(T), batch = own + (size_t)o.wrows * R * sizeof(float);
   // LDS of a workgroup: what leaves room for as many on a CU as there are (32 waves at most)
-  const int want = std::max(1, std::min((q.ntile + 255) / 256, 32 / NW));
+  const int want = std::max(1, std::min((q.ntile + 255) / 256, CH < 9 ? 32 / NW : NW == 8 ? 2 : 1));
   const int fit = (int)std::max<size_t>(1, (kLds / want - own) / batch);
   const int most = std::max(q.most, 1), pass = (most + std::min(fit, 64) - 1) / std::min(fit, 64);
   const int S = (most + pass - 1) / pass;
-  const size_t lds = std::max(own + S * batch, (size_t)NW * 64 * R * sizeof(T));
-  hipLaunchKernelGGL((k_short<T, R, NW, CH>), dim3(z.xcd ? (q.ntile + 255) / 256 * 256 : q.ntile), dim3(NW * 64), lds, st, z, S, x, y, accumulate);
+  const size_t lds = std::max(own + S * batch, (size_t)waves * 64 * R * sizeof(T));
+  hipLaunchKernelGGL((k_short<T, R, NW, CH>), dim3(z.xcd ? (q.ntile + 255) / 256 * 256 : q.ntile), dim3(waves * 64), lds, st, z, S, x, y, accumulate);
   HIP_OK(hipGetLastError());
 }
 
@@ -436,6 +443,7 @@ template <typename T, int SH>
 void launch_ch(const Owner& o, const Tab& z, const T* x, T* y, int accumulate, hipStream_t st) {
   if (o.lmax <= 64) launch<T, SH, 1>(o, z, x, y, accumulate, st);
   else if (o.lmax <= 128) launch<T, SH, 2>(o, z, x, y, accumulate, st);
+  else if (o.lmax > 256) launch<T, SH, 9>(o, z, x, y, accumulate, st);
   else launch<T, SH, 4>(o, z, x, y, accumulate, st);
 }
 
@@ -461,6 +469,11 @@ void apply_t(const Owner& o, int shape, Tab z, const T* x, T* y, int accumulate,
   z.wrows = o.wrows;
   z.ntile = q.ntile;
   z.xcd = q.ntile >= 2048;
+  z.like = shape < kPnOnly;
+  if (shape >= kPnOnly) {
+    accumulate = 1;  // after PP and NN
+    shape -= kPnOnly - 1;
+  }
   switch (shape) {
     case 0: launch_ch<T, 0>(o, z, x, y, accumulate, st); break;
     case 1: launch_ch<T, 1>(o, z, x, y, accumulate, st); break;
@@ -479,7 +492,7 @@ template <typename T, int SH>
 void allow() {
   constexpr int R = kRows[SH], NW = kWaves[SH];
   for (const void* fn : {reinterpret_cast<const void*>(k_short<T, R, NW, 1>), reinterpret_cast<const void*>(k_short<T, R, NW, 2>),
-                         reinterpret_cast<const void*>(k_short<T, R, NW, 4>)})
+                         reinterpret_cast<const void*>(k_short<T, R, NW, 4>), reinterpret_cast<const void*>(k_short<T, R, NW, 9>)})
     HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds));
 }
 
@@ -487,12 +500,13 @@ void allow() {
 
 bool Owner::has(int shape, bool f32) const {
   if (!ok || set[set_of(kRows[shape])].ntile == 0) return false;
-  if (shape >= kSplit) return f32 && pairs <= 64 && chain_lds(*this) <= kLds;
+  if (shape >= kSplit && shape < kPnOnly) return f32 && lmax <= kMaxChain && pairs <= 64 && chain_lds(*this) <= kLds;
+  if (shape >= kPnOnly && lmax <= kMaxChain / 2) return false;  // too short to pay
   return !f32 || dim >= kSplitDim;
 }
 
 int Owner::usual(bool f32) const {
-  const int q = !set[0].ntile ? 4 : set[0].ntile <= 2048 ? 2 : 1;
+  const int q = lmax > kMaxChain ? kPnOnly + 2 : !set[0].ntile ? 4 : set[0].ntile <= 2048 ? 2 : 1;
   return has(q, f32) ? q : has(kSplit + 1, f32) ? kSplit + 1 : -1;
 }
 
@@ -529,7 +543,7 @@ void build(Owner& o, const Host& h) {
   if (o.wrows > 128) return;
   o.ls = (o.lmax + 3) / 4 * 4;
   for (int v = first; v < 3; v++) {
-    const int R = 1 << v, BS = 4 + 2 * R;
+    const int R = 1 << v, BS = 6 + 2 * R;
     std::vector<Tile> tile(h.tile_f0[v].size());
     std::vector<uint32_t> batch;
     std::vector<uint32_t> pair;
@@ -548,7 +562,7 @@ void build(Owner& o, const Host& h) {
       q.nnE = (uint32_t)h.nn_emax[cn];
       q.nn = (uint32_t)h.nn_base[cn];
       q.b0 = (uint32_t)(batch.size() / BS);
-      q.q0 = (uint32_t)(pair.size() / 8);
+      q.q0 = (uint32_t)(pair.size() / 10);
       for (int k = 0; k < nd; k++) {
         int nb = 0;
         for (int r = 0; r < nr; r++) {
@@ -558,14 +572,18 @@ void build(Owner& o, const Host& h) {
         if (!nb) continue;
         const size_t ck = (size_t)cn * nd + h.negk[k];
         const uint8_t* ch = h.n1_chunk.data() + ck * 64;
-        const uint32_t E = (uint32_t)ch[0] | (uint32_t)ch[1] << 8 | (uint32_t)ch[2] << 16 | (uint32_t)ch[3] << 24;
+        uint32_t E[3];
+        for (int u = 0; u < 3; u++)
+          E[u] = (uint32_t)ch[4 * u] | (uint32_t)ch[4 * u + 1] << 8 | (uint32_t)ch[4 * u + 2] << 16 | (uint32_t)ch[4 * u + 3] << 24;
         if (h.n1q_base[ck] / 4 >= (int64_t)1 << 31) return;
-        if (!E) continue;  // no neutron jump meets it
+        if (!(E[0] | E[1] | E[2])) continue;  // no neutron jump meets it
         const int Li = h.nlen[P.conj[h.srcsec[(size_t)sp * nd + k]]];
         for (int b = 0; b < nb; b++) {
           batch.push_back((uint32_t)(h.n1q_base[ck] / 4));
           batch.push_back((uint32_t)Li | (uint32_t)h.wstride[k] << 16);
-          batch.push_back(E);
+          batch.push_back(E[0]);
+          batch.push_back(E[1]);
+          batch.push_back(E[2]);
           batch.push_back(0u);
           for (int r = 0; r < R; r++) {
             uint32_t src = kNone, wr = 0;
@@ -585,13 +603,13 @@ void build(Owner& o, const Host& h) {
           const uint32_t* rec = batch.data() + batch.size() - (size_t)nb * BS;
           for (int b = 0; b < nb; b += 2, rec += 2 * BS) {
             pair.insert(pair.end(), rec, rec + BS);
-            pair.push_back(b + 1 < nb ? rec[BS + 4] : kNone);
-            pair.push_back(b + 1 < nb ? rec[BS + 5] : 0u);
+            pair.push_back(b + 1 < nb ? rec[BS + 6] : kNone);
+            pair.push_back(b + 1 < nb ? rec[BS + 7] : 0u);
           }
         }
       }
       q.b1 = (uint32_t)(batch.size() / BS);
-      q.q1 = (uint32_t)(pair.size() / 8);
+      q.q1 = (uint32_t)(pair.size() / 10);
       if (R == 1) o.pairs = std::max(o.pairs, (int)(q.q1 - q.q0));
       most = std::max(most, (int)(q.b1 - q.b0));
     }

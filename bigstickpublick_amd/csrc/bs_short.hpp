@@ -9,12 +9,16 @@
 
 namespace bss {
 
-constexpr int kMaxRow = 256;             // longest neutron row
-// Shapes below kSplit share a column's sum among waves; the others (FP32) keep its
+constexpr int kMaxRow = 576;             // longest neutron row
+constexpr int kMaxChain = 256;           // the same for the ordered shapes
+// Shapes below kSplit share a column's sum among waves; the next two (FP32) keep its
 // order.
-constexpr int kShapes = 7, kSplit = 5;
-constexpr int kRows[kShapes] = {1, 2, 2, 4, 4, 1, 1};     // proton rows of a workgroup
-constexpr int kWaves[kShapes] = {8, 8, 16, 16, 8, 8, 16};  // its waves
+// From kPnOnly on, shapes 1 .. 4 again for the PN part alone, after the PP and NN
+// kernels (bs_like.hip).
+constexpr int kShapes = 11, kSplit = 5, kPnOnly = 7;
+constexpr int kRows[kShapes] = {1, 2, 2, 4, 4, 1, 1, 2, 2, 4, 4};        // proton rows of a workgroup
+constexpr int kWaves[kShapes] = {8, 8, 16, 16, 8, 8, 16, 8, 16, 16, 8};  // its waves
+constexpr bool ordered(int shape) { return shape >= kSplit && shape < kPnOnly; }
 // In FP32 a shared sum is rounded less often and nearer to the 64-bit one, but
 // differently.  Runs on small bases whose printed tables depend on the rounding (30
 // steps from a pivot that FP32 has let other J into: 25Mg's third digit moves)
@@ -38,10 +42,10 @@ struct Tab {
   int ntile, xcd;             // tiles; XCD-grouped order
   int ls;                     // staged row length
   int wrows;                  // coefficient rows of a batch, 2 * (largest class + 1)
-  int call_spe;
+  int call_spe, like;         // like: SPE, PP and NN too
   const Tile* tile;
   // PN batch: { neutron entry quads of (sector, class), source row length |
-  // operators << 16, entries of each 64-column chunk (a byte each), 0 } and for each
+  // operators << 16, entries of each 64-column chunk (a byte each; 3 words), 0 } and for each
   // row { source row's offset, coefficient row | negative phase << 31 } (offset
   // kNone: no jump)
   const uint32_t* batch;
@@ -98,7 +102,7 @@ struct Owner {
   // 4p4n FP32, 495 rows: two rows to 16 waves 11.2 us, to 8 waves 13.8), many rows
   // want more workgroups on a CU (pf 4p3n, 4,845 rows: 166 against 118 us); the
   // largest bases have the four-row tables alone (16 waves 527, 8 waves 433 us on pf
-  // 5p3n).  -1: none
+  // 5p3n); rows of more than 256 columns take the PN part alone.  -1: none
   int usual(bool f32) const;
   void release();
 };

@@ -120,16 +120,18 @@ int bs_apply_h(bs_system *sys, const void *x, void *y, int dtype, int accumulate
  * XCD's L2 holds their shared source rows), and prefetch (1: the next batch
  * of source rows is loaded into registers while the current one is applied;
  * 2: the same, with the proton-proton and neutron-neutron parts by kernels of
- * their own; 3: on neutron rows of at most 256 SDs, all jumps of a tile staged
- * together and a column's sum shared by 8 or (xcd_map 1) 16 waves; 4: the same
- * for one FP32 row, the sum in the order of the tile of one row and two staged
- * jumps and to its bits; FP32 has 3 from 65,536 states on).
+ * their own; 3: on neutron rows of at most 576 SDs, all jumps of a tile staged
+ * together, or as many as fit, and a column's sum shared by 8 or (xcd_map 1) 16
+ * waves; 4: the same for one FP32 row of at most 256 SDs, the sum in the order of
+ * the tile of one row and two staged jumps and to its bits; 5: the proton-neutron
+ * part of 3 after the kernels of 2, on rows of more than 128 SDs; FP32 has 3 and 5
+ * from 65,536 states on).
  * The last variant (staged = 0) is the row kernel: one thread per output
  * state, every gather from global memory, no LDS; it is the only one on
  * spaces whose neutron sectors exceed 4096 SDs or whose Delta-m operator
  * classes exceed 63 operators (up to 65535 SDs and 254 operators).
  * bs_autotune times the variants that fit in LDS on this system (those of
- * prefetch 3 and 4 alone where there are any) and keeps the fastest for that
+ * prefetch 3 to 5 alone where there are any) and keeps the fastest for that
  * dtype; bs_set_variant forces one (-1 = default choice). */
 int bs_num_variants(int *n);
 int bs_variant_info(int variant, int *rows, int *staged, int *xcd_map, int *prefetch);

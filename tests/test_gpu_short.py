@@ -1,6 +1,6 @@
 """The short-row kernel against the oracle, every shape: rows of one column, of
 fewer and of more columns than a wave and on both sides of a chunk's end, one to
-four chunks, sectors that are no multiple of a tile's rows, jumps that take more
+nine chunks, sectors that are no multiple of a tile's rows, jumps that take more
 than one pass through LDS, single-particle energies, accumulation."""
 import numpy as np
 import pytest
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("space,Z,N,jz2", [("sd", 1, 0, 1), ("sd", 2, 1, 1), ("sd", 1, 6, 1), ("sd", 3, 4, 5), ("sd", 5, 6, 1),
-                                           ("sd", 11, 6, 3), ("pf", 3, 2, 1), ("pf", 1, 3, 0), ("pf", 2, 17, 1), ("pf", 5, 2, 1)])
+                                           ("sd", 11, 6, 3), ("pf", 3, 2, 1), ("pf", 1, 3, 0), ("pf", 2, 17, 1), ("pf", 5, 2, 1), ("pf", 2, 4, 0),
+                                           ("pf", 3, 4, 3), ("pf", 1, 16, 1)])
 def test_short_rows(space, Z, N, jz2, tmp_path):
     from bigstickpublick_amd import System
     from bigstickpublick_amd.inputs import write_case
@@ -41,7 +42,7 @@ def test_short_rows(space, Z, N, jz2, tmp_path):
         xd = torch.tensor(x, device="cuda", dtype=torch.float64 if dt == "f64" else torch.float32)
         s.set_variant(dt, info.index((1, 2, 0, 0)))
         tiles = s.apply(xd)
-        ran = {3: 0, 4: 0}
+        ran = {3: 0, 4: 0, 5: 0}
         for v, i in enumerate(info):
             if i[3] < 3 or not s.set_variant(dt, v):
                 continue
@@ -53,5 +54,9 @@ def test_short_rows(space, Z, N, jz2, tmp_path):
             ya = torch.tensor(y0, device="cuda", dtype=xd.dtype)
             s.apply(xd, ya, accumulate=True)
             assert np.abs(ya.cpu().numpy()[states] - y0[states] - want).max() / scale < tol, (dt, v)
-        shared = dt == "f64" or s.dim >= 65536
-        assert ran == {3: (2 if many else 5) if shared else 0, 4: 0 if many or dt == "f64" else 2}, (dt, ran)
+        # sums shared by waves, in FP32 on bases of some size; in order, FP32 and rows of
+        # up to 256 columns; the PN part alone, from 129 columns on
+        row = (stop - start).max()
+        shared = (2 if many else 5) if dt == "f64" or s.dim >= 65536 else 0
+        alone = (2 if many else 4) if shared and row > 128 else 0
+        assert ran == {3: shared, 4: 0 if many or dt == "f64" or row > 256 else 2, 5: alone}, (dt, ran)
