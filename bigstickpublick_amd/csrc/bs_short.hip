@@ -20,6 +20,7 @@
 #include "bs_short.hpp"
 
 #include <algorithm>
+#include <cstring>
 #include <stdexcept>
 #include <string>
 
@@ -409,19 +410,38 @@ __global__ __launch_bounds__(NW * 64) void k_chain(Tab z, const float* __restric
   }
 }
 
-template <typename V>
-V* put(Owner& o, const std::vector<V>& v) {
-  void* p = nullptr;
-  HIP_OK(hipMalloc(&p, std::max<size_t>(v.size(), 1) * sizeof(V)));
-  o.mem.push_back(p);
-  if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
-  return static_cast<V*>(p);
-}
+// Tables that go to the device in one allocation and one copy
+struct Parcel {
+  std::vector<char> bytes;
+  std::vector<std::pair<void*, size_t>> at;  // address of a pointer, offset of its table
+  template <typename V>
+  void add(V** p, const std::vector<V>& v) {
+    at.push_back({p, bytes.size()});
+    const char* b = reinterpret_cast<const char*>(v.data());
+    bytes.insert(bytes.end(), b, b + v.size() * sizeof(V));
+    bytes.resize((bytes.size() / 256 + 1) * 256);
+  }
+  void send(Owner& o) {
+    void* d = nullptr;
+    HIP_OK(hipMalloc(&d, bytes.size()));
+    o.mem.push_back(d);
+    HIP_OK(hipMemcpy(d, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+    for (const auto& a : at) {
+      void* q = static_cast<char*>(d) + a.second;
+      memcpy(a.first, &q, sizeof q);
+    }
+  }
+};
 
 int set_of(int R) { return R == 1 ? 0 : R == 2 ? 1 : 2; }
 
 constexpr size_t kLds = 160 * 1024;
 constexpr size_t kManyJumps = (size_t)1 << 20, kMaxJumps = (size_t)1 << 25;
+
+// more LDS than a kernel has without asking
+void room(const void* fn, size_t lds) {
+  if (lds > 64 * 1024) HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds));
+}
 
 template <typename T, int SH, int CH>
 void launch(const Owner& o, const Tab& z, const T* x, T* y, int accumulate, hipStream_t st) {
@@ -435,6 +455,7 @@ void launch(const Owner& o, const Tab& z, const T* x, T* y, int accumulate, hipS
   const int most = std::max(q.most, 1), pass = (most + std::min(fit, 64) - 1) / std::min(fit, 64);
   const int S = (most + pass - 1) / pass;
   const size_t lds = std::max(own + S * batch, (size_t)waves * 64 * R * sizeof(T));
+  room(reinterpret_cast<const void*>(k_short<T, R, NW, CH>), lds);
   hipLaunchKernelGGL((k_short<T, R, NW, CH>), dim3(z.xcd ? (q.ntile + 255) / 256 * 256 : q.ntile), dim3(waves * 64), lds, st, z, S, x, y, accumulate);
   HIP_OK(hipGetLastError());
 }
@@ -453,6 +474,7 @@ size_t chain_lds(const Owner& o) {
 
 template <int NW>
 void launch_chain(const Owner& o, const Tab& z, const float* x, float* y, int accumulate, hipStream_t st) {
+  room(reinterpret_cast<const void*>(k_chain<NW>), chain_lds(o));
   hipLaunchKernelGGL(k_chain<NW>, dim3(o.set[0].ntile), dim3(NW * 64), chain_lds(o), st, z, x, y, accumulate);
   HIP_OK(hipGetLastError());
 }
@@ -486,14 +508,6 @@ void apply_t(const Owner& o, int shape, Tab z, const T* x, T* y, int accumulate,
         else launch_chain<16>(o, z, x, y, accumulate, st);
       }
   }
-}
-
-template <typename T, int SH>
-void allow() {
-  constexpr int R = kRows[SH], NW = kWaves[SH];
-  for (const void* fn : {reinterpret_cast<const void*>(k_short<T, R, NW, 1>), reinterpret_cast<const void*>(k_short<T, R, NW, 2>),
-                         reinterpret_cast<const void*>(k_short<T, R, NW, 4>), reinterpret_cast<const void*>(k_short<T, R, NW, 9>)})
-    HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds));
 }
 
 }  // namespace
@@ -542,6 +556,7 @@ void build(Owner& o, const Host& h) {
   o.wrows = (2 * (cmax + 1) + 3) / 4 * 4;  // (so that a batch's bytes are a multiple of 16)
   if (o.wrows > 128) return;
   o.ls = (o.lmax + 3) / 4 * 4;
+  Parcel parcel;
   for (int v = first; v < 3; v++) {
     const int R = 1 << v, BS = 6 + 2 * R;
     std::vector<Tile> tile(h.tile_f0[v].size());
@@ -615,22 +630,11 @@ void build(Owner& o, const Host& h) {
     }
     o.set[v].ntile = (int)tile.size();
     o.set[v].most = most;
-    o.set[v].tile = put(o, tile);
-    o.set[v].batch = put(o, batch);
-    if (R == 1) o.pair = put(o, pair);
+    parcel.add(&o.set[v].tile, tile);
+    parcel.add(&o.set[v].batch, batch);
+    if (R == 1) parcel.add(&o.pair, pair);
   }
-  allow<float, 0>();
-  allow<float, 1>();
-  allow<float, 2>();
-  allow<float, 3>();
-  allow<float, 4>();
-  allow<double, 0>();
-  allow<double, 1>();
-  allow<double, 2>();
-  allow<double, 3>();
-  allow<double, 4>();
-  for (const void* fn : {reinterpret_cast<const void*>(k_chain<8>), reinterpret_cast<const void*>(k_chain<16>)})
-    HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds));
+  parcel.send(o);
   o.ok = true;
 }
 
