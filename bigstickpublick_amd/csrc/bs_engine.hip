@@ -1845,6 +1845,9 @@ __global__ __launch_bounds__(1024, 4) void k_apply_lanes(DevTables tb, BatchVals
 // every system.  Same sums as k_apply_tiles: SPE, PP row AXPYs, NN ELL
 // gathers within the row, PN per proton jump over the neutron entries of the
 // conjugate class (padding slots carry the class size as operator index).
+// A slot's table reads and its gather wait for each other, so 16 slots are in flight
+// (pf 1p8n FP32 424 -> 310 us a pass; four rows of a sector to a thread, sharing a
+// slot's read, left too few waves: 542).
 template <typename T>
 __global__ __launch_bounds__(256) void k_apply_rows(DevTables tb, const int32_t* __restrict__ rows_f,
                                                     const int32_t* __restrict__ rows_c, const T* __restrict__ x,
@@ -1858,11 +1861,13 @@ __global__ __launch_bounds__(256) void k_apply_rows(DevTables tb, const int32_t*
   const int64_t bf = tb.pstart[f];
   T acc = T(0);
   if (tb.call_spe) acc = ((T)tb.pspe_sd[f] + (T)tb.nspe_sd[tb.nfirst[cn] + c]) * x[bf + c];
+#pragma unroll 4
   for (int64_t e = tb.pp_ptr[f]; e < tb.pp_ptr[f + 1]; e++)
     acc = fma(vload<T>(tb.pp_val32, tb.pp_val64, e), x[tb.pstart[tb.pp_src[e]] + c], acc);
   {
     const int64_t base = tb.nn_base[cn];
     const int E = tb.nn_emax[cn];
+#pragma unroll 16
     for (int e = 0; e < E; e++) {
       const int64_t o = base + (int64_t)e * L + c;
       acc = fma(vload<T>(tb.nn_val32, tb.nn_val64, o), x[bf + tb.nn_src[o]], acc);
@@ -1882,6 +1887,7 @@ __global__ __launch_bounds__(256) void k_apply_rows(DevTables tb, const int32_t*
       const int meta = tb.p1_meta[pj];
       const float* wr = Wk + (int64_t)(meta & 0xff) * ws;
       T a = T(0);
+#pragma unroll 4
       for (int e = 0; e < E; e++) {
         const uint32_t pk = tb.n1_pk[ebase + (int64_t)e * L + c];
         const int nl = (pk >> 16) & 0xff;
