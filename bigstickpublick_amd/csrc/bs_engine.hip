@@ -2950,6 +2950,7 @@ struct bs_system {
   DevBuf<int32_t> rows_f, rows_c;  // k_apply_rows: (proton row, first column) per workgroup
   int nrows_wg = 0;
   int variant[2] = {-1, -1};   // chosen kernel variant per dtype (0: f32, 1: f64)
+  int solve = -1;              // the FP32 variant of a solve (solve_order)
   float tune_ms[2][64] = {};    // autotuner timings (ms; 0 = not run / does not fit)
   DevTables dt{};
   DevBuf<int64_t> pstart, pp_ptr, nn_base, n1_base, n1q_base;
@@ -3603,9 +3604,9 @@ void launch_apply_v(bs_system* s, int v, const T* x, T* y, int accumulate, hipSt
 // Of the variants that one launch found within a fifth of the fastest, the one that is
 // fastest over several (a single small launch's time varies by as much): times holds
 // each one's ms, or 0.
-template <typename F>
-int settle(float* times, int n, float best, int bestv, hipEvent_t e0, hipEvent_t e1, hipStream_t st, F&& launch) {
-  auto close = [=](int v) { return times[v] > 0.0f && times[v] <= 1.2f * best; };
+template <typename W, typename F>
+int settle(float* times, int n, float best, int bestv, hipEvent_t e0, hipEvent_t e1, hipStream_t st, W&& take, F&& launch) {
+  auto close = [&](int v) { return take(v) && times[v] > 0.0f && times[v] <= 1.2f * best; };
   int some = 0;
   for (int v = 0; v < n; v++) some += close(v);
   if (best > 1.0f || some < 2) return bestv;
@@ -3625,8 +3626,39 @@ int settle(float* times, int n, float best, int bestv, hipEvent_t e0, hipEvent_t
   return bestv;
 }
 
-// Autotuner: time every variant that fits in LDS on this system (two launches
-// each on a scratch vector) and keep the fastest.
+// Order of a column's FP32 sum.  Variants of one order give the same bits: 0 adds the
+// products of one jump of a row after those of another (R1 G1, R2 G2, R4 G4), 1 those of
+// two jumps (R1 G2, R4 G2, k_chain), 2 and 3 the two and four batch slots of R2 G1 and
+// R2 G4, 4 is the row kernel's; -1: the sums that waves share (k_short) or that PP and NN
+// kernels of their own begin.
+int sum_order(int v) {
+  constexpr int kOrder[kNumShapes] = {0, 1, 2, 0, 3, 1, 0};
+  if (v == kRowsVariant) return 4;
+  if (is_short(v)) return bss::ordered(v - kShortVariant) ? 1 : -1;
+  return v < kNumVariants ? kOrder[v % kNumShapes] : -1;
+}
+
+// A solve's order.  30 Lanczos steps make some 1e-5 of FP32's rounding in one H x, so
+// Ritz vectors that have not converged, and tables printed from them, follow the order
+// of the sums and not their error: an FP32 solve keeps one order per space, by sizes and
+// not by time, and takes the fastest variant of that order.  H x by itself takes the
+// fastest of all.  The lines are where the fastest of these orders changes (timed on
+// 256 sd and pf spaces of 600 to 4.2 million states; two of them, beside a line, have
+// the next order 2% ahead or level): one-row tiles while the rows are some three
+// workgroups a CU (sd 4p5n, 495 rows: 38.7 us, R2 G4 44.3; sd 6p6n, 924 rows: 67.6 and
+// 58.4), R2 G4 up to four (pf 3p3n, 1,140 rows: 107 against R2 G2's 91), the row kernel where a row has no wave full of columns (pf 4p2n: 187 us, tiles
+// 284) or few rows are long (pf 1p6n: 211 and 219).
+int solve_order(const bs_system* s) {
+  const int64_t rows = s->dt.nP;
+  const int L = s->dt.lmax;
+  if (!s->tiles_ok) return 4;
+  if (rows > 775 && L <= (rows <= 2048 ? 4 : 64)) return 4;
+  if (rows <= 20 && L > 2048) return 4;
+  return rows <= 775 ? 1 : rows <= 1024 ? 3 : 0;
+}
+
+// Autotuner: times the variants that have a chance on this system (two launches each on
+// a scratch vector) and keeps the fastest, and in FP32 the fastest of a solve's order.
 template <typename T>
 int autotune(bs_system* s, hipStream_t st) {
   const int di = sizeof(T) == 4 ? 0 : 1;
@@ -3639,28 +3671,41 @@ int autotune(bs_system* s, hipStream_t st) {
   hipEvent_t e0, e1;
   HIP_OK(hipEventCreate(&e0));
   HIP_OK(hipEventCreate(&e1));
-  float best = 1e30f;
-  int bestv = -1;
-  for (int v = 0; v < kAllVariants; v++) {
-    if (lds_bytes<T>(s, v) > kLdsLimit) continue;
-    // on short rows no other kernel came near the short-row one's shapes
-    // (bs_short.hip: 1.3 to 4 times slower in every case)
-    if (!is_short(v) && s->brief.usual(sizeof(T) == 4) >= 0) continue;
-    // on large bases the staged-after tiles never won against the PF ones
-    // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
-    if (v < 2 * kNumShapes && s->like.ok && D >= kLikeDim) continue;
-    launch_apply_v<T>(s, v, x.p, y.p, 0, st);
+  float* ms = s->tune_ms[di];
+  std::fill(ms, ms + kAllVariants, 0.0f);
+  auto run = [&](int v) { launch_apply_v<T>(s, v, x.p, y.p, 0, st); };
+  auto time = [&](int v) {
+    run(v);
     HIP_OK(hipEventRecord(e0, st));
-    launch_apply_v<T>(s, v, x.p, y.p, 0, st);
+    run(v);
     HIP_OK(hipEventRecord(e1, st));
     HIP_OK(hipEventSynchronize(e1));
-    float ms = 0.0f;
-    HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-    s->tune_ms[di][v] = ms;
-    if (ms < best) { best = ms; bestv = v; }
+    HIP_OK(hipEventElapsedTime(&ms[v], e0, e1));
+  };
+  // of the variants that `take` names, the fastest; -1 if none of them fits
+  auto fastest = [&](auto&& take) {
+    float best = 1e30f;
+    int bestv = -1;
+    for (int v = 0; v < kAllVariants; v++) {
+      if (!take(v) || lds_bytes<T>(s, v) > kLdsLimit) continue;
+      // on large bases the staged-after tiles never won against the PF ones
+      // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
+      if (v < 2 * kNumShapes && s->like.ok && D >= kLikeDim) continue;
+      if (ms[v] == 0.0f) time(v);
+      if (ms[v] < best) { best = ms[v]; bestv = v; }
+    }
+    return settle(ms, kAllVariants, best, bestv, e0, e1, st, take, run);
+  };
+  // on short rows no other kernel came near the short-row one's shapes
+  // (bs_short.hip: 1.3 to 4 times slower in every case)
+  const bool brief = s->brief.usual(sizeof(T) == 4) >= 0;
+  const int bestv = fastest([=](int v) { return !brief || is_short(v); });
+  if (sizeof(T) == 4) {
+    const int order = solve_order(s);
+    // k_chain, where it runs, takes a third of the tiles' time
+    const bool chain = order == 1 && lds_bytes<T>(s, kShortVariant + bss::kSplit) <= kLdsLimit;
+    s->solve = fastest([=](int v) { return sum_order(v) == order && (!chain || is_short(v)); });
   }
-  bestv = settle(s->tune_ms[di], kAllVariants, best, bestv, e0, e1, st,
-                 [&](int v) { launch_apply_v<T>(s, v, x.p, y.p, 0, st); });
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (bestv < 0) throw std::runtime_error("no kernel variant fits in LDS");
@@ -3680,6 +3725,23 @@ void launch_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st
     s->variant[di] = v >= 0 ? v : kRowsVariant;
   }
   launch_apply_v<T>(s, s->variant[di], x, y, accumulate, st);
+}
+
+// y = H x as a step of a solve.  FP32: by the variant of the solve's order; until
+// autotuned, by the largest tile (order 0), or the row kernel where no tile fits.
+template <typename T>
+void launch_solve(bs_system* s, const T* x, T* y, hipStream_t st) {
+  if (sizeof(T) == 8) {
+    launch_apply<T>(s, x, y, 0, st);
+    return;
+  }
+  int v = s->solve;
+  if (v < 0) {
+    v = 2 * kNumShapes - 1;
+    while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
+    if (v < 0) v = kRowsVariant;
+  }
+  launch_apply_v<T>(s, v, x, y, 0, st);
 }
 
 // Lanczos workspace and loop
@@ -3915,7 +3977,7 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
   // against v_0 .. v_{i-1}, beta_i, v_{i+1}
   auto step = [&](int i) {
     T* vi = V.p + (int64_t)i * ld;
-    launch_apply<T>(s, vi, w.p, 0, st);
+    launch_solve<T>(s, vi, w.p, st);
     total_mv++;
     // the last nbs of part: <v_i, w>, then <w, w>; the first: the dots with V
     double* dot = part.p + (size_t)nbs * (mtot - 1);
@@ -4630,7 +4692,7 @@ int batch_variant(bs_system* s, const BatchVals& bv) {
     s->multi_ms[key][v] = ms;
     if (ms < best) { best = ms; bestv = v; }
   }
-  bestv = settle(s->multi_ms[key].data(), kNumMulti, best, bestv, e0, e1, nullptr,
+  bestv = settle(s->multi_ms[key].data(), kNumMulti, best, bestv, e0, e1, nullptr, [](int) { return true; },
                  [&](int v) { launch_batched_v<T>(s, v, bv, x.p, y.p, nullptr); });
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -5654,6 +5716,7 @@ int bs_set_variant(bs_system* s, int dtype, int v) {
       if (need > kLdsLimit) return set_err("variant does not fit in LDS for this system");
     }
     s->variant[dtype == BS_F32 ? 0 : 1] = v;
+    if (dtype == BS_F32) s->solve = v;
     return 0;
   } catch (const std::exception& e) {
     return set_err(e.what());

@@ -132,7 +132,10 @@ int bs_apply_h(bs_system *sys, const void *x, void *y, int dtype, int accumulate
  * classes exceed 63 operators (up to 65535 SDs and 254 operators).
  * bs_autotune times the variants that fit in LDS on this system (those of
  * prefetch 3 to 5 alone where there are any) and keeps the fastest for that
- * dtype; bs_set_variant forces one (-1 = default choice). */
+ * dtype; bs_set_variant forces one (-1 = default choice).  FP32 steps of
+ * bs_lanczos, bs_lanczos_noalloc and bs_strength add a column's products in an
+ * order that the space's sizes fix, and take the fastest variant of that order,
+ * or the forced one: a run's unconverged Ritz vectors follow the order. */
 int bs_num_variants(int *n);
 int bs_variant_info(int variant, int *rows, int *staged, int *xcd_map, int *prefetch);
 int bs_set_variant(bs_system *sys, int dtype, int variant);
