@@ -2927,6 +2927,8 @@ struct bs_system {
   bool kt_ready = false;               // a batch on this system holds two-row union values
   std::map<int, int> multi_choice;     // multi-vector kernel variant per (dtype, shared values, K)
   std::map<int, std::array<float, 8>> multi_ms;  // its autotuner timings
+  std::map<int, std::array<float, 8>> multi_once;  // the same of one launch each
+  std::map<int, int> multi_solve;      // a solve's variant (solve_variant)
   // adjoint tables (built on first bs_density)
   bool dens_ready = false;
   DensTables dn{};
@@ -4632,15 +4634,19 @@ void launch_ktiles(const bs_system* s, int map, const BatchVals& bv, const T* x,
   HIP_OK(hipGetLastError());
 }
 
+// one wave per basis state
+template <typename T>
+void launch_per_state(const bs_system* s, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
+  const DevTables& d = s->dt;
+  hipLaunchKernelGGL(k_apply_batched<T>, dim3(d.nP, (d.lmax + 3) / 4), dim3(256), 0, st, d, bv, x, y);
+  HIP_OK(hipGetLastError());
+}
+
 template <typename T>
 void launch_batched_v(const bs_system* s, int v, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
-  const DevTables& d = s->dt;
   if (bv.K < 1 || bv.K > kMaxBatch) throw std::runtime_error("batch size must be in 1..64");
   if (v == 0) {
-    if (launch_lanes<T>(s, bv, x, y, st)) return;
-    const int ny = (d.lmax + 3) / 4;
-    hipLaunchKernelGGL(k_apply_batched<T>, dim3(d.nP, ny), dim3(256), 0, st, d, bv, x, y);
-    HIP_OK(hipGetLastError());
+    if (!launch_lanes<T>(s, bv, x, y, st)) launch_per_state<T>(s, bv, x, y, st);
     return;
   }
   if (v >= 5) {
@@ -4657,47 +4663,107 @@ void launch_batched_v(const bs_system* s, int v, const BatchVals& bv, const T* x
   }
 }
 
+// Times launches on scratch vectors of n elements.
+template <typename T>
+struct Timer {
+  DevBuf<T> x, y;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  explicit Timer(int64_t n) {
+    x.alloc(n);
+    y.alloc(n);
+    k_fill<T><<<grid_for(n), kBlock>>>(x.p, (T)0.5, n);
+    HIP_OK(hipGetLastError());
+    HIP_OK(hipEventCreate(&e0));
+    HIP_OK(hipEventCreate(&e1));
+  }
+  ~Timer() {
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+  }
+  // ms of the second of two launches
+  template <typename F>
+  float once(F&& launch) {
+    launch(x.p, y.p);
+    HIP_OK(hipEventRecord(e0, nullptr));
+    launch(x.p, y.p);
+    HIP_OK(hipEventRecord(e1, nullptr));
+    HIP_OK(hipEventSynchronize(e1));
+    float ms = 0.0f;
+    HIP_OK(hipEventElapsedTime(&ms, e0, e1));
+    return ms;
+  }
+};
+
+// Where the tiles fit, bases from which one wave per state is two orders of magnitude
+// slower (8 s a launch on pf 6p6n) and variant 0 is not timed.
+constexpr int64_t kPerStateDim = 4000000;
+
+template <typename T>
+int multi_key(const BatchVals& bv) {
+  return (sizeof(T) == 8 ? 1000 : 0) + (bv.vk ? 0 : 100) + bv.K;
+}
+
 // The multi-vector variant for (dtype, K, shared values): timed on first use
 // (two launches each on scratch vectors) and kept.  Never called under
 // stream capture.
 template <typename T>
 int batch_variant(bs_system* s, const BatchVals& bv) {
-  const int key = (sizeof(T) == 8 ? 1000 : 0) + (bv.vk ? 0 : 100) + bv.K;
+  const int key = multi_key<T>(bv);
   auto it = s->multi_choice.find(key);
   if (it != s->multi_choice.end()) return it->second;
-  const int64_t n = s->t.dim * bv.K;
-  DevBuf<T> x, y;
-  x.alloc(n);
-  y.alloc(n);
-  k_fill<T><<<grid_for(n), kBlock>>>(x.p, (T)0.5, n);
-  HIP_OK(hipGetLastError());
-  hipEvent_t e0, e1;
-  HIP_OK(hipEventCreate(&e0));
-  HIP_OK(hipEventCreate(&e1));
+  Timer<T> tm(s->t.dim * bv.K);
   float best = 1e30f;
   int bestv = 0;
+  std::array<float, 8> ms{};
   for (int v = 0; v < kNumMulti; v++) {
     if (!multi_fits(s, v, bv.K, sizeof(T), bv.vk == 0)) continue;
-    // one wave per basis state only pays on small bases: where the tiles fit
-    // and the basis is large it is two orders of magnitude slower (8 s per
-    // launch on pf 6p6n), so it is not timed there
-    if (v == 0 && s->tiles_ok && s->t.dim > (int64_t)4000000) continue;
-    launch_batched_v<T>(s, v, bv, x.p, y.p, nullptr);
-    HIP_OK(hipEventRecord(e0, nullptr));
-    launch_batched_v<T>(s, v, bv, x.p, y.p, nullptr);
-    HIP_OK(hipEventRecord(e1, nullptr));
-    HIP_OK(hipEventSynchronize(e1));
-    float ms = 0.0f;
-    HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-    s->multi_ms[key][v] = ms;
-    if (ms < best) { best = ms; bestv = v; }
+    if (v == 0 && s->tiles_ok && s->t.dim > kPerStateDim) continue;
+    ms[v] = tm.once([&](const T* x, T* y) { launch_batched_v<T>(s, v, bv, x, y, nullptr); });
+    if (ms[v] < best) { best = ms[v]; bestv = v; }
   }
-  bestv = settle(s->multi_ms[key].data(), kNumMulti, best, bestv, e0, e1, nullptr, [](int) { return true; },
-                 [&](int v) { launch_batched_v<T>(s, v, bv, x.p, y.p, nullptr); });
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  s->multi_once[key] = ms;
+  bestv = settle(ms.data(), kNumMulti, best, bestv, tm.e0, tm.e1, nullptr, [](int) { return true; },
+                 [&](int v) { launch_batched_v<T>(s, v, bv, tm.x.p, tm.y.p, nullptr); });
+  s->multi_ms[key] = ms;
   s->multi_choice[key] = bestv;
   return bestv;
+}
+
+// The variant of a solve's steps.  As for one vector (solve_order), an FP32 solve's
+// unconverged vectors follow the order of the sums: variant 0 (either kernel) has one,
+// one staged jump (1, 2) and the two-row tiles (5, 6) another, two staged jumps (3, 4) a
+// third.  A solve keeps to the order of the fastest among the per-state and the tile
+// kernels and takes its fastest variant; k_apply_lanes, which has variant 0's bits but is
+// fast at other sizes than the per-state kernel, does not decide (sd 4p10n, K = 8 of one
+// Hamiltonian: per-state 84 us, one jump 54, two 50, lanes 46).  Never called under
+// capture.
+template <typename T>
+int solve_variant(bs_system* s, const BatchVals& bv) {
+  const int best = batch_variant<T>(s, bv);
+  if (sizeof(T) == 8) return best;
+  const int key = multi_key<T>(bv);
+  auto it = s->multi_solve.find(key);
+  if (it != s->multi_solve.end()) return it->second;
+  std::array<float, 8> once = s->multi_once[key];
+  const std::array<float, 8>& ms = s->multi_ms[key];
+  int v = best;
+  if (std::any_of(once.begin() + 1, once.end(), [](float t) { return t > 0.0f; })) {
+    if (once[0] > 0.0f) {
+      Timer<T> tm(s->t.dim * bv.K);
+      once[0] = tm.once([&](const T* x, T* y) { launch_per_state<T>(s, bv, x, y, nullptr); });
+    }
+    auto first = [](const std::array<float, 8>& t, auto&& take) {
+      int b = -1;
+      for (int q = 0; q < kNumMulti; q++)
+        if (t[q] > 0.0f && take(q) && (b < 0 || t[q] < t[b])) b = q;
+      return b;
+    };
+    constexpr int kOrder[kNumMulti] = {0, 1, 1, 2, 2, 1, 1};
+    const int order = kOrder[first(once, [](int) { return true; })];
+    v = first(ms, [&](int q) { return kOrder[q] == order; });
+  }
+  s->multi_solve[key] = v;
+  return v;
 }
 
 template <typename T>
@@ -4705,12 +4771,12 @@ void launch_batched(bs_system* s, const BatchVals& bv, const T* x, T* y, hipStre
   launch_batched_v<T>(s, batch_variant<T>(s, bv), bv, x, y, st);
 }
 
-// the chosen variant, for launches recorded under stream capture
+// the chosen variant (of a solve's step), for launches recorded under stream capture
 template <typename T>
-void launch_batched_chosen(const bs_system* s, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
-  const int key = (sizeof(T) == 8 ? 1000 : 0) + (bv.vk ? 0 : 100) + bv.K;
-  auto it = s->multi_choice.find(key);
-  if (it == s->multi_choice.end()) throw std::runtime_error("multi-vector variant not chosen before capture");
+void launch_batched_chosen(const bs_system* s, const BatchVals& bv, bool solve, const T* x, T* y, hipStream_t st) {
+  const std::map<int, int>& m = solve && sizeof(T) == 4 ? s->multi_solve : s->multi_choice;
+  auto it = m.find(multi_key<T>(bv));
+  if (it == m.end()) throw std::runtime_error("multi-vector variant not chosen before capture");
   launch_batched_v<T>(s, it->second, bv, x, y, st);
 }
 
@@ -4961,7 +5027,7 @@ int run_block_lanczos(bs_system* s, const bs_lanczos_params* p, double* evals, v
   int j = 0;
   while (true) {
     T* Vj = V.p + (int64_t)j * bsz;
-    launch_batched<T>(s, bv, Vj, W.p, st);
+    launch_batched_v<T>(s, solve_variant<T>(s, bv), bv, Vj, W.p, st);
     mv += K;
     // C_i = V_i^T W for every stored block; A_j = C_j; W -= sum_i V_i C_i
     const int m = j + 1;
@@ -5158,7 +5224,7 @@ void enqueue_batch_steps(bs_batch* b, bs_batch::Work& w, int i0, int i1, hipStre
   if (i0 == 0) k_fill<T><<<g, kBlock, 0, st>>>(V, (T)(1.0 / std::sqrt((double)D)), DK);
   for (int i = i0; i < i1; i++) {
     T* vi = V + (int64_t)i * DK;
-    launch_batched_chosen<T>(s, b->bv, vi, wv, st);
+    launch_batched_chosen<T>(s, b->bv, true, vi, wv, st);
     k_bmultidot<T><<<nb, 256, 0, st>>>(vi, DK, 1, wv, D, K, w.part.p);
     k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.alpha.p + (int64_t)i * K, 0);
     k_bsub_scaled<T><<<g, kBlock, 0, st>>>(wv, vi, w.alpha.p + (int64_t)i * K, D, K);
@@ -5341,7 +5407,7 @@ void enqueue_batch_finish(bs_batch* b, bs_batch::Work& w, int nout, hipStream_t 
     k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.dots.p, 1);
     k_bnormalize<double><<<g, kBlock, 0, st>>>(xq, xq, w.dots.p, D, K);
     if (w.polish) {
-      launch_batched_chosen<double>(s, b->bv, xq, HX, st);
+      launch_batched_chosen<double>(s, b->bv, false, xq, HX, st);
       k_bmultidot<double><<<nb, 256, 0, st>>>(xq, DK, 1, HX, D, K, w.part.p);
       k_breduce<<<1, kBReduce, 0, st>>>(w.part.p, nb, 1, K, w.rq.p + (int64_t)q * K, 0);
       k_bsub_scaled<double><<<g, kBlock, 0, st>>>(HX, xq, w.rq.p + (int64_t)q * K, D, K);
@@ -5418,7 +5484,7 @@ void run_batch_lanczos(bs_batch* b, const bs_lanczos_params* p, double* alpha, d
     w.bnorm.alloc((size_t)K);
     w.flags.alloc((size_t)K + 1);
     HIP_OK(hipStreamCreate(&w.stream));
-    batch_variant<T>(b->base.get(), b->bv);
+    solve_variant<T>(b->base.get(), b->bv);
     if (w.polish) batch_variant<double>(b->base.get(), b->bv);
     const hipStream_t st = w.stream;
     w.exec[0] = capture(st, [&] {
@@ -5970,6 +6036,7 @@ int bs_multi_variant(bs_system* s, int dtype, int K, int shared, int v) {
       return set_err("variant does not fit for this system and K");
     const int key = (dtype == BS_F64 ? 1000 : 0) + (shared ? 100 : 0) + K;
     s->multi_choice[key] = v;
+    s->multi_solve[key] = v;
     return 0;
   } catch (const std::exception& e) {
     return set_err(e.what());

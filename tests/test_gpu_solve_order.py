@@ -39,3 +39,35 @@ def test_fp32_solve_order(space, Z, N, jz2, shape, tmp_path):
     if shape != (1, 0):
         largest = solve(lambda s: s.set_variant("f32", [i[:2] for i in s.variants()].index((4, 4))))
         assert torch.equal(solve(lambda s: None)[2], largest[2])
+
+
+# K vectors: the order of the fastest among the per-state kernel (variant 0) and the
+# tile kernels (one staged jump 1, two 3), though the kernel that shares variant 0's bits
+# may be faster than the one, or slower than the other
+@pytest.mark.parametrize("what,space,Z,N,jz2,K,orders", [("block", "sd", 4, 10, 4, 8, (1, 3)), ("batch", "sd", 4, 10, 4, 8, (1, 3)),
+                                                         ("batch", "pf", 4, 1, 5, 4, (0,)), ("batch", "sd", 6, 5, 1, 3, (0,))])
+def test_fp32_k_vector_solve_order(what, space, Z, N, jz2, K, orders, tmp_path):
+    from bigstickpublick_amd import Batch, System
+    from bigstickpublick_amd.inputs import write_case
+    files = []
+    for k in range(K if what == "batch" else 1):
+        case = small_case(space, Z, N, jz2, seed=50 + k)
+        case.name += "_%d" % k
+        write_case(case, str(tmp_path))
+        files.append(paths(case, str(tmp_path)))
+
+    def solve(v):
+        if what == "batch":
+            b = Batch(files[0][0], [f[1] for f in files], Z, N, jz2)
+            assert v is None or b.set_variant("f32", v)
+            r = b.lanczos(2, 20, dtype="f32", want_vectors=True, polish=False)
+        else:
+            b = System(*files[0], Z, N, jz2, upload=True)
+            assert v is None or b.set_block_variant("f32", K, v)
+            r = b.block_lanczos(4, 6 * K, K, dtype="f32", want_vectors=True, polish=False)
+        vec = r.evecs.clone()
+        b.close()
+        return vec
+
+    got = solve(None)
+    assert any(torch.equal(got, solve(v)) for v in orders)
