@@ -2927,7 +2927,8 @@ struct bs_system {
   bool kt_ready = false;               // a batch on this system holds two-row union values
   std::map<int, int> multi_choice;     // multi-vector kernel variant per (dtype, shared values, K)
   std::map<int, std::array<float, 8>> multi_ms;  // its autotuner timings
-  std::map<int, std::array<float, 8>> multi_once;  // the same of one launch each
+  std::map<int, std::array<float, 8>> multi_once;  // of one launch each, variant 0 per state
+  std::map<int, bool> multi_per_state;   // variant 0 is the per-state kernel
   std::map<int, int> multi_solve;      // a solve's variant (solve_variant)
   // adjoint tables (built on first bs_density)
   bool dens_ready = false;
@@ -4581,6 +4582,11 @@ bool multi_fits(const bs_system* s, int v, int K, size_t tsize, bool shared) {
   return (size_t)G * K * s->dt.lmax * tsize + (size_t)kWbRows * G * K * sizeof(float) <= kLdsLimit;
 }
 
+template <typename T>
+int multi_key(const BatchVals& bv) {
+  return (sizeof(T) == 8 ? 1000 : 0) + (bv.vk ? 0 : 100) + bv.K;
+}
+
 // k_apply_lanes where its rows fit: the most groups that K and the LDS leave, with
 // two staged jumps a group if they fit; two workgroups of 8 waves on a CU, else
 // one of 16.  false: not even one group's rows fit, k_apply_batched it is.
@@ -4646,7 +4652,10 @@ template <typename T>
 void launch_batched_v(const bs_system* s, int v, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
   if (bv.K < 1 || bv.K > kMaxBatch) throw std::runtime_error("batch size must be in 1..64");
   if (v == 0) {
-    if (!launch_lanes<T>(s, bv, x, y, st)) launch_per_state<T>(s, bv, x, y, st);
+    // to the same bits: the per-state kernel where it was timed faster
+    const auto it = s->multi_per_state.find(multi_key<T>(bv));
+    if ((it != s->multi_per_state.end() && it->second) || !launch_lanes<T>(s, bv, x, y, st))
+      launch_per_state<T>(s, bv, x, y, st);
     return;
   }
   if (v >= 5) {
@@ -4698,11 +4707,6 @@ struct Timer {
 // slower (8 s a launch on pf 6p6n) and variant 0 is not timed.
 constexpr int64_t kPerStateDim = 4000000;
 
-template <typename T>
-int multi_key(const BatchVals& bv) {
-  return (sizeof(T) == 8 ? 1000 : 0) + (bv.vk ? 0 : 100) + bv.K;
-}
-
 // The multi-vector variant for (dtype, K, shared values): timed on first use
 // (two launches each on scratch vectors) and kept.  Never called under
 // stream capture.
@@ -4721,7 +4725,20 @@ int batch_variant(bs_system* s, const BatchVals& bv) {
     ms[v] = tm.once([&](const T* x, T* y) { launch_batched_v<T>(s, v, bv, x, y, nullptr); });
     if (ms[v] < best) { best = ms[v]; bestv = v; }
   }
+  // Variant 0 has two kernels of the same bits.  A workgroup of k_apply_lanes takes a
+  // proton row: with few rows most CUs have none (pf 1p4n, 20 rows, K = 34: 1,732 us,
+  // per state 207; sd 1p6n, 12 rows, K = 12: 109 and 40), with short ones a wave has no
+  // columns (pf 7p1n, rows of 1 to 4, K = 3: 6.97 ms and 3.33).  The per-state kernel is
+  // timed too, but on large bases of many rows, where it takes four times as long or more.
+  float per_state = 0.0f;
+  if (ms[0] > 0.0f && !(s->dt.nP >= 512 && s->t.dim >= 65536 && s->t.dim >= (int64_t)16 * s->dt.nP)) {
+    per_state = tm.once([&](const T* x, T* y) { launch_per_state<T>(s, bv, x, y, nullptr); });
+    s->multi_per_state[key] = per_state < ms[0];
+    ms[0] = std::min(ms[0], per_state);
+    if (ms[0] < best) { best = ms[0]; bestv = 0; }
+  }
   s->multi_once[key] = ms;
+  s->multi_once[key][0] = per_state;
   bestv = settle(ms.data(), kNumMulti, best, bestv, tm.e0, tm.e1, nullptr, [](int) { return true; },
                  [&](int v) { launch_batched_v<T>(s, v, bv, tm.x.p, tm.y.p, nullptr); });
   s->multi_ms[key] = ms;
@@ -4744,14 +4761,10 @@ int solve_variant(bs_system* s, const BatchVals& bv) {
   const int key = multi_key<T>(bv);
   auto it = s->multi_solve.find(key);
   if (it != s->multi_solve.end()) return it->second;
-  std::array<float, 8> once = s->multi_once[key];
+  const std::array<float, 8>& once = s->multi_once[key];
   const std::array<float, 8>& ms = s->multi_ms[key];
   int v = best;
   if (std::any_of(once.begin() + 1, once.end(), [](float t) { return t > 0.0f; })) {
-    if (once[0] > 0.0f) {
-      Timer<T> tm(s->t.dim * bv.K);
-      once[0] = tm.once([&](const T* x, T* y) { launch_per_state<T>(s, bv, x, y, nullptr); });
-    }
     auto first = [](const std::array<float, 8>& t, auto&& take) {
       int b = -1;
       for (int q = 0; q < kNumMulti; q++)

@@ -384,8 +384,9 @@ int bs_read_wfn(const bs_system *sys, const char *path, int first, int count, fl
 int bs_apply_block(bs_system *sys, const void *x, void *y, int K, int dtype);
 
 /* Multi-vector kernel variant for (dtype, K, shared: 1 = one Hamiltonian as
- * in bs_apply_block, 0 = one per vector as in bs_batch_apply): 0 = one wave
- * per basis state, 1..4 = one proton row per workgroup with G = 1 (1, 2) or 2
+ * in bs_apply_block, 0 = one per vector as in bs_batch_apply): 0 = one
+ * workgroup per proton row with its jumps staged, where they fit in LDS, or one
+ * wave per basis state, to the same bits (the faster where both were timed), 1..4 = one proton row per workgroup with G = 1 (1, 2) or 2
  * (3, 4) staged source rows, identity (odd) or XCD-aware (even) order; 5, 6 =
  * two proton rows per workgroup (FP32 K = 2 or 4, FP64 K = 2; one Hamiltonian
  * per vector only on a batch's system), identity (5) or XCD-aware (6) order.  Without a call the fastest is timed
