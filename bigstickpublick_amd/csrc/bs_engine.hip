@@ -2781,6 +2781,11 @@ struct DevBuf {
     alloc(v.size());
     if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   }
+  std::vector<T> download() const {
+    std::vector<T> v(n);
+    if (n) HIP_OK(hipMemcpy(v.data(), p, n * sizeof(T), hipMemcpyDeviceToHost));
+    return v;
+  }
   void release() {
     if (p && owned) (void)hipFree(p);
     p = nullptr;
@@ -2972,6 +2977,7 @@ struct bs_system {
   DevBuf<uint32_t> n1_pkr;
   DevBuf<int32_t> lane_base, lane_ptr;  // k_apply_lanes
   DevBuf<uint2> lane_ent;
+  bool lane_tried = false, lane_ok = false;
   int lane_jumps = 0;  // most jumps of a row
   DevBuf<float> pspe_sd, nspe_sd, pp_val32, nn_val32, W;
   DevBuf<double> pp_val64, nn_val64;
@@ -3337,30 +3343,7 @@ void upload_tables(bs_system* s, bool single = true) {
   s->n1_emax.upload(n1_emax);
   s->n1_pk.upload(n1_pk);
   s->n1_chunk.upload(n1_chunk);
-  {
-    // the same entries column by column, for waves that walk a column
-    std::vector<int32_t> base((size_t)N.nsec * nd), ptr;
-    std::vector<uint2> ent;
-    for (int c = 0; c < N.nsec; c++)
-      for (int k = 0; k < nd; k++) {
-        base[(size_t)c * nd + k] = (int32_t)ptr.size();
-        const uint32_t pad = (uint32_t)t.class_size[k] << 16;
-        for (int col = 0; col < nlen[c]; col++) {
-          ptr.push_back((int32_t)ent.size());
-          for (int e = 0; e < n1_emax[(size_t)c * nd + k]; e++) {
-            const uint32_t pk = n1_pk[n1_base[(size_t)c * nd + k] + (int64_t)e * nlen[c] + col];
-            if (pk == pad) continue;
-            ent.push_back(make_uint2((pk & 0xffffffu) | ((pk >> 24 & 1u) << 31), (uint32_t)col));
-          }
-          if ((int32_t)ent.size() > ptr.back()) ent.back().y |= 1u << 31;
-        }
-        ptr.push_back((int32_t)ent.size());
-      }
-    for (int f = 0; f < nP; f++) s->lane_jumps = std::max(s->lane_jumps, pcls[(size_t)f * (nd + 1) + nd] - pcls[(size_t)f * (nd + 1)]);
-    s->lane_base.upload(base);
-    s->lane_ptr.upload(ptr);
-    s->lane_ent.upload(ent);
-  }
+  for (int f = 0; f < nP; f++) s->lane_jumps = std::max(s->lane_jumps, pcls[(size_t)f * (nd + 1) + nd] - pcls[(size_t)f * (nd + 1)]);
   {
     std::vector<uint32_t> v(n1_pk.size());
     for (size_t i = 0; i < n1_pk.size(); i++) {
@@ -4589,26 +4572,79 @@ int multi_key(const BatchVals& bv) {
 
 // k_apply_lanes where its rows fit: the most groups that K and the LDS leave, with
 // two staged jumps a group if they fit; two workgroups of 8 waves on a CU, else
-// one of 16.  false: not even one group's rows fit, k_apply_batched it is.
+// one of 16.  H = 0: not even one group's rows fit, k_apply_batched it is.
+struct LaneShape {
+  int H, G;
+  size_t bytes;
+};
+LaneShape lane_shape(const bs_system* s, int K, int size) {
+  const DevTables& d = s->dt;
+  if (d.lmax > 4096 || d.dim > (int64_t)UINT32_MAX) return {0, 0, 0};
+  auto lds = [&](int H, int G) {
+    return (size_t)LaneLds(H, G, size, d.lmax * K, (d.wcols - 1) * K, s->lane_jumps, d.ndelta).bytes;
+  };
+  int H = K <= 8 ? 8 : K <= 16 ? 4 : K <= 32 ? 2 : 1;
+  while (H > 1 && lds(H, 1) > kLdsLimit) H /= 2;
+  if (lds(H, 1) > kLdsLimit) return {0, 0, 0};
+  const int G = lds(H, 2) <= kLdsLimit ? 2 : 1;
+  return {H, G, lds(H, G)};
+}
+
+// The neutron one-body entries column by column, when K vectors of `size` bytes an
+// element first want them (8 bytes an entry; a lone vector never does).  Where memory
+// for them runs out the per-state kernel goes on alone.  Never called under capture.
+void want_lanes(bs_system* s, int K, int size) {
+  if (s->lane_tried || !lane_shape(s, K, size).H) return;
+  s->lane_tried = true;
+  try {
+    const std::vector<uint32_t> pk = s->n1_pk.download();
+    const std::vector<int64_t> pk0 = s->n1_base.download();
+    const std::vector<int32_t> emax = s->n1_emax.download(), nlen = s->nlen.download();
+    const int nd = s->t.ndelta, nsec = s->t.sp[1].nsec;
+    std::vector<int32_t> base((size_t)nsec * nd), ptr;
+    std::vector<uint2> ent;
+    for (int c = 0; c < nsec; c++)
+      for (int k = 0; k < nd; k++) {
+        const size_t ck = (size_t)c * nd + k;
+        base[ck] = (int32_t)ptr.size();
+        const uint32_t pad = (uint32_t)s->t.class_size[k] << 16;
+        for (int col = 0; col < nlen[c]; col++) {
+          ptr.push_back((int32_t)ent.size());
+          for (int e = 0; e < emax[ck]; e++) {
+            const uint32_t q = pk[pk0[ck] + (int64_t)e * nlen[c] + col];
+            if (q == pad) continue;
+            ent.push_back(make_uint2((q & 0xffffffu) | ((q >> 24 & 1u) << 31), (uint32_t)col));
+          }
+          if ((int32_t)ent.size() > ptr.back()) ent.back().y |= 1u << 31;
+        }
+        ptr.push_back((int32_t)ent.size());
+      }
+    s->lane_base.upload(base);
+    s->lane_ptr.upload(ptr);
+    s->lane_ent.upload(ent);
+    s->lane_ok = true;
+  } catch (const std::exception&) {
+    (void)hipGetLastError();
+    s->lane_base.release();
+    s->lane_ptr.release();
+    s->lane_ent.release();
+  }
+}
+
 template <typename T>
 bool launch_lanes(const bs_system* s, const BatchVals& bv, const T* x, T* y, hipStream_t st) {
   const DevTables& d = s->dt;
-  if (d.lmax > 4096 || d.dim > (int64_t)UINT32_MAX) return false;
-  auto lds = [&](int H, int G) {
-    return (size_t)LaneLds(H, G, (int)sizeof(T), d.lmax * bv.K, (d.wcols - 1) * bv.K, s->lane_jumps, d.ndelta).bytes;
-  };
-  int H = bv.K <= 8 ? 8 : bv.K <= 16 ? 4 : bv.K <= 32 ? 2 : 1;
-  while (H > 1 && lds(H, 1) > kLdsLimit) H /= 2;
-  if (lds(H, 1) > kLdsLimit) return false;
-  const int G = lds(H, 2) <= kLdsLimit ? 2 : 1;
-  const int threads = lds(H, G) <= kLdsLimit / 2 ? 512 : 1024;
+  const LaneShape q = lane_shape(s, bv.K, (int)sizeof(T));
+  if (!q.H || !s->lane_ok) return false;
+  const int H = q.H, G = q.G;
+  const int threads = q.bytes <= kLdsLimit / 2 ? 512 : 1024;
   constexpr int V = 16 / (int)sizeof(T);
   const bool vec = bv.K % V == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
   const LaneTables lt{s->lane_base.p, s->lane_ptr.p, s->lane_ent.p, s->lane_jumps};
   auto go = [&](auto fn) {
     HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)kLdsLimit));
-    hipLaunchKernelGGL(fn, dim3(d.nP), dim3(threads), lds(H, G), st, d, bv, lt, x, y);
+    hipLaunchKernelGGL(fn, dim3(d.nP), dim3(threads), q.bytes, st, d, bv, lt, x, y);
     HIP_OK(hipGetLastError());
   };
 #define BS_LANES(HH, GG) \
@@ -4715,6 +4751,7 @@ int batch_variant(bs_system* s, const BatchVals& bv) {
   const int key = multi_key<T>(bv);
   auto it = s->multi_choice.find(key);
   if (it != s->multi_choice.end()) return it->second;
+  want_lanes(s, bv.K, (int)sizeof(T));
   Timer<T> tm(s->t.dim * bv.K);
   float best = 1e30f;
   int bestv = 0;
@@ -6047,6 +6084,7 @@ int bs_multi_variant(bs_system* s, int dtype, int K, int shared, int v) {
     if (v < 0 || v >= kNumMulti) return set_err("no such multi-vector variant");
     if (!multi_fits(s, v, K, dtype == BS_F32 ? 4 : 8, shared != 0))
       return set_err("variant does not fit for this system and K");
+    if (v == 0) want_lanes(s, K, dtype == BS_F32 ? 4 : 8);
     const int key = (dtype == BS_F64 ? 1000 : 0) + (shared ? 100 : 0) + K;
     s->multi_choice[key] = v;
     s->multi_solve[key] = v;
