@@ -2781,9 +2781,10 @@ struct DevBuf {
     alloc(v.size());
     if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   }
-  std::vector<T> download() const {
+  std::vector<T> download(hipStream_t st = nullptr) const {
     std::vector<T> v(n);
-    if (n) HIP_OK(hipMemcpy(v.data(), p, n * sizeof(T), hipMemcpyDeviceToHost));
+    if (n) HIP_OK(hipMemcpyAsync(v.data(), p, n * sizeof(T), hipMemcpyDeviceToHost, st));
+    HIP_OK(hipStreamSynchronize(st));
     return v;
   }
   void release() {
@@ -2959,6 +2960,7 @@ struct bs_system {
   int nrows_wg = 0;
   int variant[2] = {-1, -1};   // chosen kernel variant per dtype (0: f32, 1: f64)
   int solve = -1;              // the FP32 variant of a solve (solve_order)
+  int ran[2] = {-1, -1};       // the variant last run while none was chosen
   float tune_ms[2][64] = {};    // autotuner timings (ms; 0 = not run / does not fit)
   DevTables dt{};
   DevBuf<int64_t> pstart, pp_ptr, nn_base, n1_base, n1q_base;
@@ -2981,8 +2983,13 @@ struct bs_system {
   int lane_jumps = 0;  // most jumps of a row
   DevBuf<float> pspe_sd, nspe_sd, pp_val32, nn_val32, W;
   DevBuf<double> pp_val64, nn_val64;
-  bsl::Owner like;              // tables of the separate PP and NN kernels
-  bss::Owner brief;             // tables of the short-row kernel
+  // Tables of the separate PP and NN kernels and of the short-row kernel (want_tables)
+  bool lone = true;             // not a batch's system, which has no use for them
+  std::mutex want;
+  std::atomic<bool> wanted[2] = {{false}, {false}};  // built, or found not to be buildable
+  bool brief_tried = false;
+  bsl::Owner like;
+  bss::Owner brief;
 };
 
 namespace {
@@ -3020,9 +3027,7 @@ void order_by_operator(uint32_t* pk, int L, int em, uint32_t pad) {
   }
 }
 
-// single: the tables of the separate PP and NN kernels and of the short-row kernel
-// too, which a batch has no use for
-void upload_tables(bs_system* s, bool single = true) {
+void upload_tables(bs_system* s) {
   const bs::Tables& t = s->t;
   const bs::Species& P = t.sp[0];
   const bs::Species& N = t.sp[1];
@@ -3211,10 +3216,8 @@ void upload_tables(bs_system* s, bool single = true) {
     if (P.start[f] < 0 || P.start[f] + nlen[P.conj[P.sdsec[f]]] > t.dim) throw std::runtime_error("row outside the vector");
   // tiles for each R, and two workgroup->tile maps: identity (sector order)
   // and XCD-grouped (below)
-  std::vector<int32_t> tile_f0[3], tile_nr[3];
-  std::vector<int64_t> tpp_ptr[3];
   for (int v = 0; v < 3; v++) {
-    std::vector<int32_t>&f0 = tile_f0[v], &nr = tile_nr[v];
+    std::vector<int32_t> f0, nr;
     for (int sp = 0; sp < P.nsec; sp++)
       for (int64_t f = P.secfirst[sp]; f < P.secfirst[sp] + P.seccount[sp]; f += kTileRows[v]) {
         f0.push_back((int32_t)f);
@@ -3228,8 +3231,7 @@ void upload_tables(bs_system* s, bool single = true) {
       // PP source union per tile (sources of all R rows, each listed once)
       const int R = kTileRows[v];
       const bs::TwoBody& T = t.tb[0];
-      std::vector<int64_t>& ptr = tpp_ptr[v];
-      ptr.assign(nt + 1, 0);
+      std::vector<int64_t> ptr(nt + 1, 0);
       std::vector<uint32_t> src;
       std::vector<float> v32;
       std::vector<double> v64;
@@ -3439,10 +3441,6 @@ void upload_tables(bs_system* s, bool single = true) {
   d.wrows = s->wrows.p;
   d.wstride = s->wstride.p;
   d.negk = s->negk.p;
-  if (s->tiles_ok && single) bsl::build(s->like, t, s->pstart.p, s->psec.p, s->pconj.p, s->nlen.p, nlen, s->pp_ptr.p, s->pp_src.p, s->pp_val64.p);
-  if (s->tiles_ok && single)
-    bss::build(s->brief, {t, nlen, srcsec, pcls, p1_src, p1_meta, n1q_base, n1_chunk, nn_base, nn_emax, woff, wstride, negk,
-                          tile_f0, tile_nr, tpp_ptr});
   s->uploaded = true;
 }
 
@@ -3519,10 +3517,57 @@ template <typename T>
 size_t lds_bytes(const bs_system* s, int v) {
   if (v == kRowsVariant) return 0;
   if (!s->tiles_ok) return SIZE_MAX;
-  if (is_short(v))
-    return s->brief.has(v - kShortVariant, sizeof(T) == 4) && (v - kShortVariant < bss::kPnOnly || s->like.ok) ? 0 : SIZE_MAX;
-  if (is_like(v) && !s->like.ok) return SIZE_MAX;
+  if (is_short(v) || is_like(v)) {
+    constexpr int di = sizeof(T) == 4 ? 0 : 1;
+    if (!s->wanted[di].load(std::memory_order_acquire)) return SIZE_MAX;
+    if (is_short(v))
+      return s->brief.has(v - kShortVariant, sizeof(T) == 4) && (v - kShortVariant < bss::kPnOnly || s->like.ok[di]) ? 0 : SIZE_MAX;
+    if (!s->like.ok[di]) return SIZE_MAX;
+  }
   return lds_bytes_rg<T>(s, kVarR[v % kNumShapes], kVarG[v % kNumShapes]);
+}
+
+// The tables of the separate PP and NN kernels (with the values of T) and of the
+// short-row kernel, when H x by itself first wants them: block, gradient and batch
+// passes, operators applied once and FP32 solves on long rows never read them (pf 4p4n:
+// a third of the upload).  Where memory for them runs out, the tiles go on alone.  On a
+// stream of its own, and not counted against a capture under way on another thread;
+// never called under capture on this one.
+template <typename T>
+void want_tables(bs_system* s) {
+  constexpr int di = sizeof(T) == 4 ? 0 : 1;
+  if (s->wanted[di].load(std::memory_order_acquire)) return;
+  std::lock_guard<std::mutex> lock(s->want);
+  if (s->wanted[di].load(std::memory_order_relaxed)) return;
+  if (s->lone && s->tiles_ok) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_OK(hipThreadExchangeStreamCaptureMode(&mode));
+    hipStream_t st = nullptr;
+    try {
+      HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+      const std::vector<int32_t> nlen = s->nlen.download(st);
+      if (!s->brief_tried) {
+        s->brief_tried = true;
+        if (*std::max_element(nlen.begin(), nlen.end()) <= bss::kMaxRow) {
+          const std::vector<int32_t> f0[3] = {s->tile_f0[0].download(st), s->tile_f0[1].download(st), s->tile_f0[2].download(st)};
+          const std::vector<int32_t> nr[3] = {s->tile_nr[0].download(st), s->tile_nr[1].download(st), s->tile_nr[2].download(st)};
+          const std::vector<int64_t> pp[3] = {s->tpp_ptr[0].download(st), s->tpp_ptr[1].download(st), s->tpp_ptr[2].download(st)};
+          bss::build(s->brief, {s->t, nlen, s->srcsec.download(st), s->pcls.download(st), s->p1_src.download(st),
+                                s->p1_meta.download(st), s->n1q_base.download(st), s->n1_chunk.download(st),
+                                s->nn_base.download(st), s->nn_emax.download(st), s->woff.download(st),
+                                s->wstride.download(st), s->negk.download(st), f0, nr, pp}, st);
+        }
+      }
+      bsl::build(s->like, {s->t, nlen, s->pstart.p, s->psec.p, s->pconj.p, s->nlen.p, s->pp_ptr.p, s->pp_src.p, s->pp_val64.p},
+                 sizeof(T) == 4, st);
+    } catch (const std::exception&) {
+      (void)hipGetLastError();
+      if (!s->brief.ok) s->brief.release();
+    }
+    if (st) (void)hipStreamDestroy(st);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  s->wanted[di].store(true, std::memory_order_release);
 }
 
 template <typename T, int CPT>
@@ -3649,6 +3694,7 @@ template <typename T>
 int autotune(bs_system* s, hipStream_t st) {
   const int di = sizeof(T) == 4 ? 0 : 1;
   const int64_t D = s->t.dim;
+  want_tables<T>(s);
   DevBuf<T> x, y;
   x.alloc(D);
   y.alloc(D);
@@ -3676,7 +3722,7 @@ int autotune(bs_system* s, hipStream_t st) {
       if (!take(v) || lds_bytes<T>(s, v) > kLdsLimit) continue;
       // on large bases the staged-after tiles never won against the PF ones
       // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
-      if (v < 2 * kNumShapes && s->like.ok && D >= kLikeDim) continue;
+      if (v < 2 * kNumShapes && s->like.ok[di] && D >= kLikeDim) continue;
       if (ms[v] == 0.0f) time(v);
       if (ms[v] < best) { best = ms[v]; bestv = v; }
     }
@@ -3684,7 +3730,7 @@ int autotune(bs_system* s, hipStream_t st) {
   };
   // on short rows no other kernel came near the short-row one's shapes
   // (bs_short.hip: 1.3 to 4 times slower in every case)
-  const bool brief = s->brief.usual(sizeof(T) == 4) >= 0;
+  const bool brief = s->brief.usual(sizeof(T) == 4, s->like.ok[di]) >= 0;
   const int bestv = fastest([=](int v) { return !brief || is_short(v); });
   if (sizeof(T) == 4) {
     const int order = solve_order(s);
@@ -3699,33 +3745,54 @@ int autotune(bs_system* s, hipStream_t st) {
   return bestv;
 }
 
+// Until autotuned or told: on short rows a shape of their kernel, on large bases the
+// largest tile with the separate PP and NN kernels, if their tables are there; else the
+// largest tile that fits.
 template <typename T>
-void launch_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st) {
-  const int di = sizeof(T) == 4 ? 0 : 1;
-  if (s->variant[di] < 0) {
-    // until autotuned: on short rows a shape of their kernel; else the largest
-    // tile that fits, on large bases with the separate PP and NN kernels
-    const int sh = s->brief.usual(sizeof(T) == 4);
-    int v = sh >= 0 ? kShortVariant + sh : s->like.ok && s->t.dim >= kLikeDim ? kShortVariant - 1 : 2 * kNumShapes - 1;
-    while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
-    s->variant[di] = v >= 0 ? v : kRowsVariant;
+int default_variant(const bs_system* s) {
+  constexpr int di = sizeof(T) == 4 ? 0 : 1;
+  int v = 2 * kNumShapes - 1;
+  if (s->wanted[di].load(std::memory_order_acquire)) {
+    const int sh = s->brief.usual(sizeof(T) == 4, s->like.ok[di]);
+    if (sh >= 0) v = kShortVariant + sh;
+    else if (s->like.ok[di] && s->t.dim >= kLikeDim) v = kShortVariant - 1;
   }
-  launch_apply_v<T>(s, s->variant[di], x, y, accumulate, st);
+  while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
+  return v >= 0 ? v : kRowsVariant;
 }
 
-// y = H x as a step of a solve.  FP32: by the variant of the solve's order; until
-// autotuned, by the largest tile (order 0), or the row kernel where no tile fits.
+template <typename T>
+void launch_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st) {
+  constexpr int di = sizeof(T) == 4 ? 0 : 1;
+  int v = s->variant[di];
+  if (v < 0) s->ran[di] = v = default_variant<T>(s);
+  launch_apply_v<T>(s, v, x, y, accumulate, st);
+}
+
+// A caller's H x: with every table, but under capture, where nothing can be built.
+template <typename T>
+void caller_apply(bs_system* s, const T* x, T* y, int accumulate, hipStream_t st) {
+  if (s->variant[sizeof(T) == 4 ? 0 : 1] < 0) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) != hipSuccess) (void)hipGetLastError();  // (the launch will tell)
+    else if (c == hipStreamCaptureStatusNone) want_tables<T>(s);
+  }
+  launch_apply<T>(s, x, y, accumulate, st);
+}
+
+// y = H x as a step of a solve.  FP32: by the variant of the solve's order.  Until
+// autotuned, in either type, by the largest tile, or the row kernel where no tile fits,
+// whichever tables H x by itself has had built: a solve's bits are not to follow the
+// calls before it, nor whether it may allocate (bs_lanczos_noalloc).
 template <typename T>
 void launch_solve(bs_system* s, const T* x, T* y, hipStream_t st) {
-  if (sizeof(T) == 8) {
-    launch_apply<T>(s, x, y, 0, st);
-    return;
-  }
-  int v = s->solve;
+  constexpr int di = sizeof(T) == 4 ? 0 : 1;
+  int v = di == 0 ? s->solve : s->variant[1];
   if (v < 0) {
     v = 2 * kNumShapes - 1;
     while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
     if (v < 0) v = kRowsVariant;
+    s->ran[di] = v;
   }
   launch_apply_v<T>(s, v, x, y, 0, st);
 }
@@ -4182,7 +4249,7 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
       k_reduce<<<1, kBlock, 0, st>>>(part.p, nb, 1, dots.p, 1);
       k_normalize<double><<<g, kBlock, 0, st>>>(xk, xk, dots.p, D);
       if (p->polish || resid) {
-        launch_apply<double>(s, xk, HX.p, 0, st);
+        launch_solve<double>(s, xk, HX.p, st);
         total_mv++;
         k_multidot<double><<<nb, kBlock, 0, st>>>(xk, D, 1, HX.p, D, part.p);
         k_reduce<<<1, kBlock, 0, st>>>(part.p, nb, 1, dots.p + 1, 0);
@@ -5211,7 +5278,7 @@ int run_block_lanczos(bs_system* s, const bs_lanczos_params* p, double* evals, v
       k_reduce<<<1, kBlock, 0, st>>>(part1.p, nb1, 1, dots.p, 1);
       k_normalize<double><<<g, kBlock, 0, st>>>(xk, xk, dots.p, D);
       if (p->polish || resid) {
-        launch_apply<double>(s, xk, HX.p, 0, st);
+        launch_solve<double>(s, xk, HX.p, st);
         mv++;
         k_multidot<double><<<nb1, kBlock, 0, st>>>(xk, D, 1, HX.p, D, part1.p);
         k_reduce<<<1, kBlock, 0, st>>>(part1.p, nb1, 1, dots.p + 1, 0);
@@ -5779,8 +5846,8 @@ int bs_apply_h(bs_system* s, const void* x, void* y, int dtype, int accumulate, 
     if (!x || !y) return set_err("null vector");
     if (x == y) return set_err("x and y must not overlap");
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == BS_F32) launch_apply<float>(s, (const float*)x, (float*)y, accumulate ? 1 : 0, st);
-    else if (dtype == BS_F64) launch_apply<double>(s, (const double*)x, (double*)y, accumulate ? 1 : 0, st);
+    if (dtype == BS_F32) caller_apply<float>(s, (const float*)x, (float*)y, accumulate ? 1 : 0, st);
+    else if (dtype == BS_F64) caller_apply<double>(s, (const double*)x, (double*)y, accumulate ? 1 : 0, st);
     else return set_err("dtype must be BS_F32 or BS_F64");
     return 0;
   } catch (const std::exception& e) {
@@ -5828,10 +5895,12 @@ int bs_set_variant(bs_system* s, int dtype, int v) {
     if (dtype != BS_F32 && dtype != BS_F64) return set_err("dtype must be BS_F32 or BS_F64");
     if (v < -1 || v >= kAllVariants) return set_err("bad variant");
     if (v >= 0) {
+      if (is_short(v) || is_like(v)) dtype == BS_F32 ? want_tables<float>(s) : want_tables<double>(s);
       size_t need = dtype == BS_F32 ? lds_bytes<float>(s, v) : lds_bytes<double>(s, v);
       if (need > kLdsLimit) return set_err("variant does not fit in LDS for this system");
     }
     s->variant[dtype == BS_F32 ? 0 : 1] = v;
+    s->ran[dtype == BS_F32 ? 0 : 1] = -1;
     if (dtype == BS_F32) s->solve = v;
     return 0;
   } catch (const std::exception& e) {
@@ -5841,7 +5910,8 @@ int bs_set_variant(bs_system* s, int dtype, int v) {
 
 int bs_get_variant(const bs_system* s, int dtype, int* v) {
   if (!s || !v || (dtype != BS_F32 && dtype != BS_F64)) return set_err("bad argument");
-  *v = s->variant[dtype == BS_F32 ? 0 : 1];
+  const int di = dtype == BS_F32 ? 0 : 1;
+  *v = s->variant[di] < 0 ? s->ran[di] : s->variant[di];
   return 0;
 }
 
@@ -5873,8 +5943,8 @@ int bs_apply_h_host(bs_system* s, const void* x, void* y, int dtype, int accumul
     }
     HIP_OK(hipMemcpy(s->hostx.p, x, bytes, hipMemcpyHostToDevice));
     if (accumulate) HIP_OK(hipMemcpy(s->hosty.p, y, bytes, hipMemcpyHostToDevice));
-    if (dtype == BS_F32) launch_apply<float>(s, (const float*)s->hostx.p, (float*)s->hosty.p, accumulate ? 1 : 0, nullptr);
-    else launch_apply<double>(s, (const double*)s->hostx.p, (double*)s->hosty.p, accumulate ? 1 : 0, nullptr);
+    if (dtype == BS_F32) caller_apply<float>(s, (const float*)s->hostx.p, (float*)s->hosty.p, accumulate ? 1 : 0, nullptr);
+    else caller_apply<double>(s, (const double*)s->hostx.p, (double*)s->hosty.p, accumulate ? 1 : 0, nullptr);
     HIP_OK(hipMemcpy(y, s->hosty.p, bytes, hipMemcpyDeviceToHost));
     return 0;
   } catch (const std::exception& e) {
@@ -6127,7 +6197,8 @@ int bs_batch_init(const char* sps, const char* const* intfiles, int K, int Z, in
     bs::ModelInput in;
     bs::read_sps(sps, in);
     b->base->t = bs::build_tables_structural(in.orbits, intfiles[0], Z, N, jz2, spscale, a0, a, x);
-    upload_tables(b->base.get(), false);
+    b->base->lone = false;
+    upload_tables(b->base.get());
     batch_upload_values(b.get());
     HIP_OK(hipDeviceSynchronize());
     *out = b.release();
@@ -6457,7 +6528,7 @@ int bs_exact(bs_system* s, int nkeep, int dtype, double* evals, void* evecs, dou
       double* xk = Hd.p + (int64_t)k * D;
       if (resid) {
         // ||H x - E x|| of the eigenvector, one more apply
-        launch_apply<double>(s, xk, HX.p, 0, st);
+        launch_solve<double>(s, xk, HX.p, st);
         HIP_OK(hipMemcpy(dots.p + 1, &evals[k], sizeof(double), hipMemcpyHostToDevice));
         k_sub_scaled<double><<<gd, kBlock, 0, st>>>(HX.p, xk, dots.p + 1, D);
         k_multidot<double><<<nb1, kBlock, 0, st>>>(HX.p, D, 1, HX.p, D, part1.p);

@@ -263,7 +263,7 @@ __global__ __launch_bounds__(1024) void k_nn(Tab z, const T* __restrict__ x, T* 
 // A[block][lane][step] of the PP tiles from the merged entries by row
 __global__ __launch_bounds__(256) void k_pp_fill(int ntile, const int32_t* row0, const int32_t* tnr, const int32_t* tblk,
                                                  const int32_t* usrc, const int64_t* pp_ptr, const int32_t* pp_src,
-                                                 const double* pp_val, float* A32, double* A64) {
+                                                 const double* pp_val, float* A32, double* A64) {  // (one of A32, A64)
   const int t = blockIdx.x;
   const int b0 = tblk[t], n = (tblk[t + 1] - b0) * 16;
   const int32_t* u = usrc + (int64_t)b0 * 16;
@@ -278,10 +278,10 @@ __global__ __launch_bounds__(256) void k_pp_fill(int ntile, const int32_t* row0,
       }
       const int64_t blk = b0 + lo / 16;
       const int s = lo % 16 / 4, lk = lo % 4;
-      A32[(blk * 64 + lk * 16 + r) * 4 + s] = (float)pp_val[e];
+      if (A32) A32[(blk * 64 + lk * 16 + r) * 4 + s] = (float)pp_val[e];
       // FP64 result register i of lane group g is matrix row g + 4 i
       const int i = r / 4 + 4 * (r % 4);
-      A64[((blk * 2 + s / 2) * 64 + lk * 16 + i) * 2 + s % 2] = pp_val[e];
+      if (A64) A64[((blk * 2 + s / 2) * 64 + lk * 16 + i) * 2 + s % 2] = pp_val[e];
     }
   }
 }
@@ -289,14 +289,18 @@ __global__ __launch_bounds__(256) void k_pp_fill(int ntile, const int32_t* row0,
 template <typename V>
 V* get(Owner& o, size_t n) {
   void* p = nullptr;
+  o.mem.reserve(o.mem.size() + 1);
   HIP_OK(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(V)));
   o.mem.push_back(p);
   return static_cast<V*>(p);
 }
 template <typename V>
-V* put(Owner& o, const std::vector<V>& v) {
+V* put(Owner& o, const std::vector<V>& v, hipStream_t st) {
   V* p = get<V>(o, v.size());
-  if (!v.empty()) HIP_OK(hipMemcpy(p, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice));
+  if (!v.empty()) {
+    HIP_OK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(V), hipMemcpyHostToDevice, st));
+    HIP_OK(hipStreamSynchronize(st));
+  }
   return p;
 }
 
@@ -315,14 +319,17 @@ void parallel(int n, F&& body) {
 
 template <typename T>
 void apply_t(const Owner& o, const T* x, T* y, int accumulate, hipStream_t st) {
-  if (!o.ok) throw std::runtime_error("like-particle tables missing");
+  if (!o.ok[sizeof(T) == 4 ? 0 : 1]) throw std::runtime_error("like-particle tables missing");
+  Tab z = o.t;
+  if constexpr (sizeof(T) == 4) z.pA32 = o.pA32, z.nval32 = o.nval32;
+  else z.pA64 = o.pA64, z.nval64 = o.nval64;
   constexpr int C = sizeof(T) == 4 ? 4096 : 2048;
   const int nw = std::min(16, (o.lmax + 63) / 64);
   const size_t lds = (size_t)std::min(o.lmax, C) * kNnRows * sizeof(T);
-  hipLaunchKernelGGL(k_nn<T>, dim3((o.t.nnn + 255) / 256 * 256), dim3(64 * nw), lds, st, o.t, x, y, accumulate);
+  hipLaunchKernelGGL(k_nn<T>, dim3((o.t.nnn + 255) / 256 * 256), dim3(64 * nw), lds, st, z, x, y, accumulate);
   HIP_OK(hipGetLastError());
   if (o.t.npp > 0) {
-    k_pp<<<o.t.npp, 256, 0, st>>>(o.t, x, y);
+    k_pp<<<o.t.npp, 256, 0, st>>>(z, x, y);
     HIP_OK(hipGetLastError());
   }
 }
@@ -332,22 +339,38 @@ void apply_t(const Owner& o, const T* x, T* y, int accumulate, hipStream_t st) {
 void Owner::release() {
   for (void* p : mem) (void)hipFree(p);
   mem.clear();
-  ok = false;
+  ok[0] = ok[1] = false;
+  ntile = 0;
 }
 
 void apply(const Owner& o, const float* x, float* y, int accumulate, hipStream_t st) { apply_t<float>(o, x, y, accumulate, st); }
 void apply(const Owner& o, const double* x, double* y, int accumulate, hipStream_t st) { apply_t<double>(o, x, y, accumulate, st); }
 
-void build(Owner& o, const bs::Tables& t, const int64_t* pstart, const int32_t* psec, const int32_t* pconj,
-           const int32_t* nlen, const std::vector<int32_t>& nlen_h, const int64_t* pp_ptr, const int32_t* pp_src,
-           const double* pp_val) {
-  o.release();
+namespace {
+
+// entries of the neutron columns n0 .. n0 + nl of one half (source columns below 2048 of
+// the sector, from 2048 on): [lo, hi) of each, and the most of one
+int half_entries(const bs::TwoBody& nn, int64_t sec, int64_t n0, int nl, int h, int64_t* lo, int64_t* hi) {
+  int most = 0;
+  for (int l = 0; l < nl; l++) {
+    const auto b = nn.src.begin() + nn.rowptr[n0 + l], e = nn.src.begin() + nn.rowptr[n0 + l + 1];
+    const auto m = std::lower_bound(b, e, (int32_t)(sec + 2048));
+    lo[l] = (h ? m : b) - nn.src.begin();
+    hi[l] = (h ? e : m) - nn.src.begin();
+    most = std::max(most, (int)(hi[l] - lo[l]));
+  }
+  return most;
+}
+
+bool structure(Owner& o, const Host& g, hipStream_t st) {
+  const bs::Tables& t = g.t;
+  const std::vector<int32_t>& nlen_h = g.nlen_h;
   const bs::Species& P = t.sp[0];
   const bs::Species& N = t.sp[1];
   const int nP = (int)P.mask.size();
   int lmax = 0;
   for (int c : nlen_h) lmax = std::max(lmax, c);
-  if (lmax < 1 || lmax > 4096 || t.call_spe || nP < 1) return;
+  if (lmax < 1 || lmax > 4096 || t.call_spe || nP < 1) return false;
   // PP tiles: 16 rows of a sector, the union of their sources in blocks of 16
   std::vector<int32_t> row0, tnr, tL, tfirst, tblk(1, 0);
   std::vector<int64_t> tsec;
@@ -355,7 +378,7 @@ void build(Owner& o, const bs::Tables& t, const int64_t* pstart, const int32_t* 
   for (int s = 0; s < P.nsec; s++) {
     const int L = nlen_h[P.conj[s]];
     const int64_t el = P.seccount[s] * L;
-    if (el * 8 >= (int64_t)1 << 31) return;  // a sector is addressed with 32-bit byte offsets
+    if (el * 8 >= (int64_t)1 << 31) return false;  // a sector is addressed with 32-bit byte offsets
     for (int64_t f = 0; f < P.seccount[s]; f += kPpRows) {
       row0.push_back((int32_t)(P.secfirst[s] + f));
       tnr.push_back((int32_t)std::min<int64_t>(kPpRows, P.seccount[s] - f));
@@ -411,75 +434,102 @@ void build(Owner& o, const bs::Tables& t, const int64_t* pstart, const int32_t* 
       nnr.push_back((int32_t)std::min<int64_t>(kNnRows, P.seccount[s] - f));
     }
   std::vector<uint32_t> nng((size_t)N.nsec * 128, 0), nsrc;
-  std::vector<double> nval;
+  int64_t lo[64], hi[64];
   for (int c = 0; c < N.nsec; c++)
     for (int cc = 0; cc * 64 < nlen_h[c]; cc++)
       for (int h = 0; h < 2; h++) {
-        const int64_t n0 = N.secfirst[c] + cc * 64;
         const int nl = std::min(64, nlen_h[c] - cc * 64);
-        int most = 0;
-        int64_t lo[64], hi[64];
-        for (int l = 0; l < nl; l++) {
-          const auto b = t.tb[1].src.begin() + t.tb[1].rowptr[n0 + l], e = t.tb[1].src.begin() + t.tb[1].rowptr[n0 + l + 1];
-          const auto m = std::lower_bound(b, e, (int32_t)(N.secfirst[c] + 2048));
-          lo[l] = (h ? m : b) - t.tb[1].src.begin();
-          hi[l] = (h ? e : m) - t.tb[1].src.begin();
-          most = std::max(most, (int)(hi[l] - lo[l]));
-        }
-        const int np = (most + 3) / 4 * 2;
-        if (np > 1023) return;
+        const int np = (half_entries(t.tb[1], N.secfirst[c], N.secfirst[c] + cc * 64, nl, h, lo, hi) + 3) / 4 * 2;
+        if (np > 1023) return false;
         const size_t o0 = nsrc.size() / 64;
-        if (o0 >= (1u << 22)) return;
+        if (o0 >= (1u << 22)) return false;
         nng[((size_t)c * 64 + cc) * 2 + h] = (uint32_t)o0 << 10 | (uint32_t)np;
         // padding entries: value zero at the chunk's first source column
         nsrc.resize(nsrc.size() + (size_t)np * 64, 0u);
-        nval.resize(nval.size() + (size_t)np * 128, 0.0);
         for (int l = 0; l < nl; l++)
           for (int64_t q = lo[l]; q < hi[l]; q++) {
             const int i = (int)(q - lo[l]);
             const uint32_t sc = (uint32_t)(t.tb[1].src[q] - N.secfirst[c]) - 2048u * h;
             nsrc[(o0 + i / 2) * 64 + l] |= sc << (16 * (i % 2));
-            nval[(o0 * 2 + i) * 64 + l] = t.tb[1].val[q];
           }
       }
-  std::vector<float> nvalf(nval.begin(), nval.end());
   Tab& d = o.t;
+  d = Tab{};
   d.npp = (int)pitem.size();
   d.nnn = (int)nf0.size();
-  d.pitem = put(o, pitem);
-  d.tsec = put(o, tsec);
-  d.tbytes = put(o, tbytes);
-  d.tfirst = put(o, tfirst);
-  d.tnr = put(o, tnr);
-  d.tL = put(o, tL);
-  d.tblk = put(o, tblk);
-  d.psrc = put(o, psrc);
-  const size_t na = (size_t)tblk.back() * 256;
-  float* A32 = get<float>(o, na);
-  double* A64 = get<double>(o, na);
-  HIP_OK(hipMemset(A32, 0, std::max<size_t>(na, 1) * sizeof(float)));
-  HIP_OK(hipMemset(A64, 0, std::max<size_t>(na, 1) * sizeof(double)));
-  int32_t* d_row0 = put(o, row0);
-  int32_t* d_usrc = put(o, usrc);
-  k_pp_fill<<<nt, 256>>>(nt, d_row0, d.tnr, d.tblk, d_usrc, pp_ptr, pp_src, pp_val, A32, A64);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipDeviceSynchronize());
-  d.pA32 = A32;
-  d.pA64 = A64;
-  d.nf0 = put(o, nf0);
-  d.nnr = put(o, nnr);
-  d.psec = psec;
-  d.pconj = pconj;
-  d.nlen = nlen;
-  d.pstart = pstart;
-  d.nng = put(o, nng);
-  d.nsrc = put(o, nsrc);
-  d.nval32 = put(o, nvalf);
-  d.nval64 = put(o, nval);
+  d.pitem = put(o, pitem, st);
+  d.tsec = put(o, tsec, st);
+  d.tbytes = put(o, tbytes, st);
+  d.tfirst = put(o, tfirst, st);
+  d.tnr = put(o, tnr, st);
+  d.tL = put(o, tL, st);
+  d.tblk = put(o, tblk, st);
+  d.psrc = put(o, psrc, st);
+  d.nf0 = put(o, nf0, st);
+  d.nnr = put(o, nnr, st);
+  d.psec = g.psec;
+  d.pconj = g.pconj;
+  d.nlen = g.nlen;
+  d.pstart = g.pstart;
+  d.nng = put(o, nng, st);
+  d.nsrc = put(o, nsrc, st);
+  o.row0 = put(o, row0, st);
+  o.usrc = put(o, usrc, st);
+  o.blocks = tblk.back();
+  o.nrows = (int64_t)nsrc.size() / 64;
+  o.nng = std::move(nng);
   o.lmax = lmax;
   for (const void* fn : {reinterpret_cast<const void*>(k_nn<float>), reinterpret_cast<const void*>(k_nn<double>)})
     HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-  o.ok = true;
+  o.ntile = nt;
+  return true;
+}
+
+// the PP coefficients and the NN values of one type
+template <typename T>
+void values(Owner& o, const Host& g, const T** pA, const T** nval, hipStream_t st) {
+  const bs::Species& N = g.t.sp[1];
+  const size_t na = std::max<size_t>((size_t)o.blocks * 256, 1);
+  T* A = get<T>(o, na);
+  HIP_OK(hipMemsetAsync(A, 0, na * sizeof(T), st));
+  if constexpr (sizeof(T) == 4)
+    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.row0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, A, nullptr);
+  else
+    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.row0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, nullptr, A);
+  HIP_OK(hipGetLastError());
+  std::vector<T> v((size_t)o.nrows * 128, T(0));
+  int64_t lo[64], hi[64];
+  for (int c = 0; c < N.nsec; c++)
+    for (int cc = 0; cc * 64 < g.nlen_h[c]; cc++)
+      for (int h = 0; h < 2; h++) {
+        const int nl = std::min(64, g.nlen_h[c] - cc * 64);
+        half_entries(g.t.tb[1], N.secfirst[c], N.secfirst[c] + cc * 64, nl, h, lo, hi);
+        T* at = v.data() + (size_t)(o.nng[((size_t)c * 64 + cc) * 2 + h] >> 10) * 128;
+        for (int l = 0; l < nl; l++)
+          for (int64_t q = lo[l]; q < hi[l]; q++) at[(q - lo[l]) * 64 + l] = (T)g.t.tb[1].val[q];
+      }
+  *nval = put(o, v, st);  // (waits for k_pp_fill too)
+  HIP_OK(hipStreamSynchronize(st));
+  *pA = A;
+}
+
+}  // namespace
+
+void build(Owner& o, const Host& g, bool f32, hipStream_t st) {
+  if (o.ok[f32 ? 0 : 1]) return;
+  const size_t had = o.mem.size();
+  try {
+    if (!o.ntile && !structure(o, g, st)) return;
+    if (f32) values<float>(o, g, &o.pA32, &o.nval32, st);
+    else values<double>(o, g, &o.pA64, &o.nval64, st);
+    o.ok[f32 ? 0 : 1] = true;
+  } catch (...) {  // the other type keeps what it has
+    (void)hipStreamSynchronize(st);
+    for (size_t i = had; i < o.mem.size(); i++) (void)hipFree(o.mem[i]);
+    o.mem.resize(had);
+    if (!had) o.ntile = 0;
+    throw;
+  }
 }
 
 }  // namespace bsl

@@ -44,17 +44,37 @@ struct Tab {
 };
 
 struct Owner {
-  bool ok = false;
+  bool ok[2] = {false, false};  // tables and values of FP32, FP64
   int lmax = 0;
-  Tab t{};
+  Tab t{};                      // without the values
+  const float *pA32 = nullptr, *nval32 = nullptr;
+  const double *pA64 = nullptr, *nval64 = nullptr;
+  int ntile = 0;                // PP tiles, their first rows and sources, for the values
+  int64_t blocks = 0, nrows = 0;
+  const int32_t* row0 = nullptr;
+  const int32_t* usrc = nullptr;
+  std::vector<uint32_t> nng;
   std::vector<void*> mem;
   ~Owner() { release(); }
   void release();
 };
 
-void build(Owner& o, const bs::Tables& t, const int64_t* pstart, const int32_t* psec, const int32_t* pconj,
-           const int32_t* nlen, const std::vector<int32_t>& nlen_h, const int64_t* pp_ptr, const int32_t* pp_src,
-           const double* pp_val);
+// What build() reads of the engine's tables (the pointers: on the device)
+struct Host {
+  const bs::Tables& t;
+  const std::vector<int32_t>& nlen_h;
+  const int64_t* pstart;
+  const int32_t* psec;
+  const int32_t* pconj;
+  const int32_t* nlen;
+  const int64_t* pp_ptr;
+  const int32_t* pp_src;
+  const double* pp_val;
+};
+
+// Tables with the values of one type; the other type's are added by a second call.
+// Device work goes to `st`, which is waited for.
+void build(Owner& o, const Host& h, bool f32, hipStream_t st);
 
 // y (+)= (H_pp + H_nn) x
 void apply(const Owner& o, const float* x, float* y, int accumulate, hipStream_t st);

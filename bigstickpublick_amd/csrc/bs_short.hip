@@ -421,11 +421,13 @@ struct Parcel {
     bytes.insert(bytes.end(), b, b + v.size() * sizeof(V));
     bytes.resize((bytes.size() / 256 + 1) * 256);
   }
-  void send(Owner& o) {
+  void send(Owner& o, hipStream_t st) {
     void* d = nullptr;
+    o.mem.reserve(1);
     HIP_OK(hipMalloc(&d, bytes.size()));
     o.mem.push_back(d);
-    HIP_OK(hipMemcpy(d, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpyAsync(d, bytes.data(), bytes.size(), hipMemcpyHostToDevice, st));
+    HIP_OK(hipStreamSynchronize(st));
     for (const auto& a : at) {
       void* q = static_cast<char*>(d) + a.second;
       memcpy(a.first, &q, sizeof q);
@@ -519,8 +521,8 @@ bool Owner::has(int shape, bool f32) const {
   return !f32 || dim >= kSplitDim;
 }
 
-int Owner::usual(bool f32) const {
-  const int q = lmax > kMaxChain ? kPnOnly + 2 : !set[0].ntile ? 4 : set[0].ntile <= 2048 ? 2 : 1;
+int Owner::usual(bool f32, bool like) const {
+  const int q = lmax > kMaxChain && like ? kPnOnly + 2 : !set[0].ntile ? 4 : set[0].ntile <= 2048 ? 2 : 1;
   return has(q, f32) ? q : has(kSplit + 1, f32) ? kSplit + 1 : -1;
 }
 
@@ -538,7 +540,7 @@ void apply(const Owner& o, int shape, Tab z, const double* x, double* y, int acc
   apply_t<double>(o, shape, z, x, y, accumulate, st);
 }
 
-void build(Owner& o, const Host& h) {
+void build(Owner& o, const Host& h, hipStream_t st) {
   o.release();
   const bs::Species& P = h.t.sp[0];
   const bs::Species& N = h.t.sp[1];
@@ -634,7 +636,7 @@ void build(Owner& o, const Host& h) {
     parcel.add(&o.set[v].batch, batch);
     if (R == 1) parcel.add(&o.pair, pair);
   }
-  parcel.send(o);
+  parcel.send(o, st);
   o.ok = true;
 }
 

@@ -102,12 +102,14 @@ struct Owner {
   // 4p4n FP32, 495 rows: two rows to 16 waves 11.2 us, to 8 waves 13.8), many rows
   // want more workgroups on a CU (pf 4p3n, 4,845 rows: 166 against 118 us); the
   // largest bases have the four-row tables alone (16 waves 527, 8 waves 433 us on pf
-  // 5p3n); rows of more than 256 columns take the PN part alone.  -1: none
-  int usual(bool f32) const;
+  // 5p3n); rows of more than 256 columns take the PN part alone if the PP
+  // and NN kernels can run (like).  -1: none
+  int usual(bool f32, bool like) const;
   void release();
 };
 
-void build(Owner& o, const Host& h);
+// device work goes to `st`, which is waited for
+void build(Owner& o, const Host& h, hipStream_t st);
 
 // y (+)= H x by shape 0 .. kShapes - 1; z holds the engine's tables for its R
 // (tiles, batches and LDS strides are filled in)
