@@ -2986,8 +2986,7 @@ struct bs_system {
   // Tables of the separate PP and NN kernels and of the short-row kernel (want_tables)
   bool lone = true;             // not a batch's system, which has no use for them
   std::mutex want;
-  std::atomic<bool> wanted[2] = {{false}, {false}};  // built, or found not to be buildable
-  bool brief_tried = false;
+  std::atomic<bool> brief_tried{false}, like_tried[2] = {{false}, {false}};  // built, or cannot be
   bsl::Owner like;
   bss::Owner brief;
 };
@@ -3500,7 +3499,7 @@ void launch_variant(bs_system* s, int map, bool pf, const T* x, T* y, int accumu
 // The separate kernels read a PP source row once per 16 target rows on the
 // matrix cores and an NN entry once per 8 rows, which the tile kernel's LDS and
 // registers have no room for (pf 6p6n: 2.9 + 1.5 ms FP32, 5.4 + 2.8 ms FP64).
-// They pay from rows of some hundred columns on (pf 4p4n FP32 549 -> 464 us, and 319
+// They pay from some hundred proton rows of some hundred columns on (pf 4p4n FP32 549 -> 464 us, and 319
 // with the PN part by k_short;
 // pf 6p6n 21.0 -> 18.9 ms, FP64 42.7 -> 35.2 ms); on short rows the two extra
 // launches and the tiles' padding cost more (pf 2p3n 32 -> 68 us).
@@ -3513,61 +3512,81 @@ constexpr int64_t kLikeDim = 1000000;  // basis size from which they are the def
 constexpr bool is_like(int v) { return v >= kLikeVariant && v < kShortVariant; }
 constexpr bool is_short(int v) { return v >= kShortVariant && v < kRowsVariant; }
 
+// the separate PP and NN kernels can run
+template <typename T>
+bool like_ok(const bs_system* s) {
+  constexpr int di = sizeof(T) == 4 ? 0 : 1;
+  return s->like_tried[di].load(std::memory_order_acquire) && s->like.ok[di];
+}
+
+// the usual shape of the short-row kernel, -1 where it cannot run
+template <typename T>
+int brief_usual(const bs_system* s) {
+  return s->brief_tried.load(std::memory_order_acquire) ? s->brief.usual(sizeof(T) == 4, like_ok<T>(s)) : -1;
+}
+
 template <typename T>
 size_t lds_bytes(const bs_system* s, int v) {
   if (v == kRowsVariant) return 0;
   if (!s->tiles_ok) return SIZE_MAX;
   if (is_short(v) || is_like(v)) {
-    constexpr int di = sizeof(T) == 4 ? 0 : 1;
-    if (!s->wanted[di].load(std::memory_order_acquire)) return SIZE_MAX;
-    if (is_short(v))
-      return s->brief.has(v - kShortVariant, sizeof(T) == 4) && (v - kShortVariant < bss::kPnOnly || s->like.ok[di]) ? 0 : SIZE_MAX;
-    if (!s->like.ok[di]) return SIZE_MAX;
+    if (is_short(v)) {
+      if (!s->brief_tried.load(std::memory_order_acquire) || !s->brief.has(v - kShortVariant, sizeof(T) == 4)) return SIZE_MAX;
+      if (v - kShortVariant < bss::kPnOnly) return 0;
+    }
+    if (!like_ok<T>(s)) return SIZE_MAX;
+    if (is_short(v)) return 0;
   }
   return lds_bytes_rg<T>(s, kVarR[v % kNumShapes], kVarG[v % kNumShapes]);
 }
 
-// The tables of the separate PP and NN kernels (with the values of T) and of the
-// short-row kernel, when H x by itself first wants them: block, gradient and batch
-// passes, operators applied once and FP32 solves on long rows never read them (pf 4p4n:
-// a third of the upload).  Where memory for them runs out, the tiles go on alone.  On a
-// stream of its own, and not counted against a capture under way on another thread;
-// never called under capture on this one.
+// The tables of the short-row kernel and of the separate PP and NN kernels (with the
+// values of T), when H x by itself first wants them: block, gradient and batch passes,
+// operators applied once and solves that are not tuned never read them (pf 4p4n: half
+// of the upload).  PP and NN tables only where their kernels pay, or are asked for by
+// name: on few proton rows they gain a few percent for a table time of some hundred
+// passes (pf 1p5n, 20 rows: 89 -> 83 us for 10 ms; pf 3p5n, 1,140 rows: 290 -> 254 us),
+// on rows of up to 128 columns they lose.  Where memory runs out, the tiles go on alone.
+// On a stream of its own, and not counted against a capture under way on another
+// thread; never called under capture on this one.
 template <typename T>
-void want_tables(bs_system* s) {
+void want_tables(bs_system* s, bool named = false) {
   constexpr int di = sizeof(T) == 4 ? 0 : 1;
-  if (s->wanted[di].load(std::memory_order_acquire)) return;
+  if (!s->lone || !s->tiles_ok) return;
+  const bool like = named || (s->dt.nP >= 512 && s->dt.lmax > 128);
+  auto done = [&]() {
+    return s->brief_tried.load(std::memory_order_acquire) && (!like || s->like_tried[di].load(std::memory_order_acquire));
+  };
+  if (done()) return;
   std::lock_guard<std::mutex> lock(s->want);
-  if (s->wanted[di].load(std::memory_order_relaxed)) return;
-  if (s->lone && s->tiles_ok) {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    HIP_OK(hipThreadExchangeStreamCaptureMode(&mode));
-    hipStream_t st = nullptr;
-    try {
-      HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-      const std::vector<int32_t> nlen = s->nlen.download(st);
-      if (!s->brief_tried) {
-        s->brief_tried = true;
-        if (*std::max_element(nlen.begin(), nlen.end()) <= bss::kMaxRow) {
-          const std::vector<int32_t> f0[3] = {s->tile_f0[0].download(st), s->tile_f0[1].download(st), s->tile_f0[2].download(st)};
-          const std::vector<int32_t> nr[3] = {s->tile_nr[0].download(st), s->tile_nr[1].download(st), s->tile_nr[2].download(st)};
-          const std::vector<int64_t> pp[3] = {s->tpp_ptr[0].download(st), s->tpp_ptr[1].download(st), s->tpp_ptr[2].download(st)};
-          bss::build(s->brief, {s->t, nlen, s->srcsec.download(st), s->pcls.download(st), s->p1_src.download(st),
-                                s->p1_meta.download(st), s->n1q_base.download(st), s->n1_chunk.download(st),
-                                s->nn_base.download(st), s->nn_emax.download(st), s->woff.download(st),
-                                s->wstride.download(st), s->negk.download(st), f0, nr, pp}, st);
-        }
-      }
+  if (done()) return;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIP_OK(hipThreadExchangeStreamCaptureMode(&mode));
+  hipStream_t st = nullptr;
+  try {
+    HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    const std::vector<int32_t> nlen = s->nlen.download(st);
+    if (!s->brief_tried && *std::max_element(nlen.begin(), nlen.end()) <= bss::kMaxRow) {
+      const std::vector<int32_t> f0[3] = {s->tile_f0[0].download(st), s->tile_f0[1].download(st), s->tile_f0[2].download(st)};
+      const std::vector<int32_t> nr[3] = {s->tile_nr[0].download(st), s->tile_nr[1].download(st), s->tile_nr[2].download(st)};
+      const std::vector<int64_t> pp[3] = {s->tpp_ptr[0].download(st), s->tpp_ptr[1].download(st), s->tpp_ptr[2].download(st)};
+      bss::build(s->brief, {s->t, nlen, s->srcsec.download(st), s->pcls.download(st), s->p1_src.download(st),
+                            s->p1_meta.download(st), s->n1q_base.download(st), s->n1_chunk.download(st),
+                            s->nn_base.download(st), s->nn_emax.download(st), s->woff.download(st),
+                            s->wstride.download(st), s->negk.download(st), f0, nr, pp}, st);
+    }
+    s->brief_tried.store(true, std::memory_order_release);
+    if (like)
       bsl::build(s->like, {s->t, nlen, s->pstart.p, s->psec.p, s->pconj.p, s->nlen.p, s->pp_ptr.p, s->pp_src.p, s->pp_val64.p},
                  sizeof(T) == 4, st);
-    } catch (const std::exception&) {
-      (void)hipGetLastError();
-      if (!s->brief.ok) s->brief.release();
-    }
-    if (st) (void)hipStreamDestroy(st);
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  } catch (const std::exception&) {
+    (void)hipGetLastError();
+    if (!s->brief_tried) s->brief.release();
   }
-  s->wanted[di].store(true, std::memory_order_release);
+  if (st) (void)hipStreamDestroy(st);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  s->brief_tried.store(true, std::memory_order_release);
+  if (like) s->like_tried[di].store(true, std::memory_order_release);
 }
 
 template <typename T, int CPT>
@@ -3640,7 +3659,7 @@ int settle(float* times, int n, float best, int bestv, hipEvent_t e0, hipEvent_t
   auto close = [&](int v) { return take(v) && times[v] > 0.0f && times[v] <= 1.2f * best; };
   int some = 0;
   for (int v = 0; v < n; v++) some += close(v);
-  if (best > 1.0f || some < 2) return bestv;
+  if (best > 0.05f || some < 2) return bestv;  // (longer launches vary by a percent or two)
   float least = 1e30f;
   for (int v = 0; v < n; v++) {
     if (!close(v)) continue;
@@ -3722,7 +3741,7 @@ int autotune(bs_system* s, hipStream_t st) {
       if (!take(v) || lds_bytes<T>(s, v) > kLdsLimit) continue;
       // on large bases the staged-after tiles never won against the PF ones
       // (pf 6p6n, R4 G4: 23.1 against 21.0 ms)
-      if (v < 2 * kNumShapes && s->like.ok[di] && D >= kLikeDim) continue;
+      if (v < 2 * kNumShapes && like_ok<T>(s) && D >= kLikeDim) continue;
       if (ms[v] == 0.0f) time(v);
       if (ms[v] < best) { best = ms[v]; bestv = v; }
     }
@@ -3730,7 +3749,7 @@ int autotune(bs_system* s, hipStream_t st) {
   };
   // on short rows no other kernel came near the short-row one's shapes
   // (bs_short.hip: 1.3 to 4 times slower in every case)
-  const bool brief = s->brief.usual(sizeof(T) == 4, s->like.ok[di]) >= 0;
+  const bool brief = brief_usual<T>(s) >= 0;
   const int bestv = fastest([=](int v) { return !brief || is_short(v); });
   if (sizeof(T) == 4) {
     const int order = solve_order(s);
@@ -3750,13 +3769,8 @@ int autotune(bs_system* s, hipStream_t st) {
 // largest tile that fits.
 template <typename T>
 int default_variant(const bs_system* s) {
-  constexpr int di = sizeof(T) == 4 ? 0 : 1;
-  int v = 2 * kNumShapes - 1;
-  if (s->wanted[di].load(std::memory_order_acquire)) {
-    const int sh = s->brief.usual(sizeof(T) == 4, s->like.ok[di]);
-    if (sh >= 0) v = kShortVariant + sh;
-    else if (s->like.ok[di] && s->t.dim >= kLikeDim) v = kShortVariant - 1;
-  }
+  const int sh = brief_usual<T>(s);
+  int v = sh >= 0 ? kShortVariant + sh : like_ok<T>(s) && s->t.dim >= kLikeDim ? kShortVariant - 1 : 2 * kNumShapes - 1;
   while (v >= 0 && lds_bytes<T>(s, v) > kLdsLimit) v--;
   return v >= 0 ? v : kRowsVariant;
 }
@@ -5895,7 +5909,7 @@ int bs_set_variant(bs_system* s, int dtype, int v) {
     if (dtype != BS_F32 && dtype != BS_F64) return set_err("dtype must be BS_F32 or BS_F64");
     if (v < -1 || v >= kAllVariants) return set_err("bad variant");
     if (v >= 0) {
-      if (is_short(v) || is_like(v)) dtype == BS_F32 ? want_tables<float>(s) : want_tables<double>(s);
+      if (is_short(v) || is_like(v)) dtype == BS_F32 ? want_tables<float>(s, true) : want_tables<double>(s, true);
       size_t need = dtype == BS_F32 ? lds_bytes<float>(s, v) : lds_bytes<double>(s, v);
       if (need > kLdsLimit) return set_err("variant does not fit in LDS for this system");
     }
