@@ -2947,6 +2947,7 @@ struct bs_system {
   DevBuf<int64_t> d_pn_toff;
   DevBuf<uint16_t> d_pn_tgt;
   bool dens_lds = false;       // the PN pass stages rows in LDS
+  bool dens_gather = false;    // it gathers from memory also where they fit (bs_set_density_gather)
   std::vector<int32_t> nn_comp_to_me;
   bool jac_ready = false;
   std::vector<bs::ParamColumn> jac;
@@ -4392,7 +4393,7 @@ void build_density_tables(bs_system* s) {
   const int mc1 = t.max_class + 1;
   int lmax = 0;
   for (int c = 0; c < N.nsec; c++) lmax = std::max<int>(lmax, (int)N.seccount[c]);
-  s->dens_lds = lmax < 0x7fff && ((size_t)lmax + 1) * sizeof(double) <= kLdsLimit;
+  s->dens_lds = !s->dens_gather && lmax < 0x7fff && ((size_t)lmax + 1) * sizeof(double) <= kLdsLimit;
   std::vector<int64_t> poff, toff((size_t)N.nsec * nd, 0);
   std::vector<std::vector<uint64_t>> bucket(mc1);
   std::vector<uint64_t> ppk;
@@ -6073,6 +6074,13 @@ int bs_num_params(const bs_system* s, int* nspe, int* ntbme) {
   if (!s) return set_err("null system");
   if (nspe) *nspe = (int)s->t.in.orbits.size();
   if (ntbme) *ntbme = (int)s->t.lines.size();
+  return 0;
+}
+
+int bs_set_density_gather(bs_system* s, int on) {
+  if (!s) return set_err("null system");
+  if (s->dens_gather != (on != 0)) s->dens_ready = false;
+  s->dens_gather = on != 0;
   return 0;
 }
 

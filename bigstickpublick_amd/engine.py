@@ -62,6 +62,7 @@ def load_library():
     L.bs_num_params.argtypes = [vp, ctypes.POINTER(i32), ctypes.POINTER(i32)]
     L.bs_density.argtypes = [vp, vp, i32, vp, vp, vp, ctypes.POINTER(ctypes.c_double)]
     L.bs_gradient.argtypes = [vp, vp, i32, vp]
+    L.bs_set_density_gather.argtypes = [vp, i32]
     L.bs_observable.argtypes = [vp, i32, vp, i32, ctypes.POINTER(ctypes.c_double)]
     L.bs_lanczos.argtypes = [vp, ctypes.POINTER(_Params), vp, vp, vp, vp, vp,
                              ctypes.POINTER(i32)]
@@ -338,6 +339,11 @@ class System:
         _check(load_library().bs_density(self.h, ctypes.c_void_p(psi.data_ptr()), dt, rpp.ctypes.data,
                                          rnn.ctypes.data, rpn.ctypes.data, ctypes.byref(n2)))
         return rpp, rnn, rpn, n2.value
+
+    def set_density_gather(self, on):
+        """The proton-neutron density by gathers from memory, as on rows over
+        20,479 SDs, also where the rows fit in LDS."""
+        _check(load_library().bs_set_density_gather(self.h, int(on)))
 
     def gradient(self, psi):
         """dE/dtheta for theta = (SPEs, TBME lines in .int order), psi a CUDA vector."""

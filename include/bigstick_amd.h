@@ -171,6 +171,11 @@ int bs_num_params(const bs_system *sys, int *nspe, int *ntbme);
 int bs_density(bs_system *sys, const void *psi, int dtype, double *rho_pp, double *rho_nn,
                double *rho_pn, double *norm2);
 
+/* on = 1: bs_density and bs_gradient take the proton-neutron part by gathers
+ * from memory, as on neutron rows over 20,479 SDs, also where the rows fit in
+ * LDS (0, the default).  Builds the density tables anew. */
+int bs_set_density_gather(bs_system *sys, int on);
+
 /* Hellmann-Feynman gradient dE/dtheta = <psi|dH/dtheta|psi>/<psi|psi> for all
  * interaction parameters (grad has nspe + ntbme entries, order of
  * bs_num_params), from bs_density and the Jacobian of the FP32 elements with
