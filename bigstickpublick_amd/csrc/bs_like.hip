@@ -42,6 +42,33 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, uint32_
 // columns 4 (l % 16) .. + 3 (FP32; FP64: 2 (l % 16), + 1 and 32 further), and
 // feeds v_mfma_*_16x16x4 once per column: result register r is row
 // 4 (l / 16) + r of the tile (FP64: the matrix rows are permuted for that).
+// A zero of the union times an infinity is NaN: a result that is not finite is
+// left out and summed over its row's own entries instead (again), so that a
+// source that is not finite reaches the rows that H connects it to and no others.
+// sets results that are not finite to zero: bit 4 i + u is column u of row i
+template <typename V>
+__device__ __forceinline__ uint32_t take_out(V (&d)[4]) {
+  uint32_t out = 0;
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (!isfinite(d[u][i])) {
+        out |= 1u << (4 * i + u);
+        d[u][i] = 0;
+      }
+  return out;
+}
+
+// yrow[col] += proton SD f's sum over its own entries
+template <typename T>
+__device__ __forceinline__ void again(const Tab& z, const T* __restrict__ x, T* __restrict__ yrow, int64_t f, int col) {
+  T s = T(0);
+  for (int64_t e = z.pp_ptr[f]; e < z.pp_ptr[f + 1]; e++)
+    s = fma((T)z.pp_val[e], x[z.pstart[z.pp_src[e]] + col], s);
+  yrow[col] += s;
+}
+
 __global__ __launch_bounds__(256) void k_pp(Tab z, const float* __restrict__ x, float* __restrict__ y) {
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint64_t it = cst(z.pitem)[blockIdx.x];
@@ -85,6 +112,7 @@ __global__ __launch_bounds__(256) void k_pp(Tab z, const float* __restrict__ x, 
       for (int u = 0; u < 4; u++) d[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(ac[q], xv[q][u], d[u], 0, 0, 0);
   }
   const int nr = cst(z.tnr)[t], f0 = cst(z.tfirst)[t];
+  uint32_t out = take_out(d);
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int row = 4 * lk + i;
@@ -101,6 +129,11 @@ __global__ __launch_bounds__(256) void k_pp(Tab z, const float* __restrict__ x, 
           if (cl + u >= c && cl + u < L) o[u] += d[u][i];
       }
     }
+  }
+  for (; out; out &= out - 1) {
+    const int q = __builtin_ctz(out), row = 4 * lk + (q >> 2), col = cl + (q & 3);
+    if (row < nr && col >= c && col < L)
+      again(z, x, y + sec + (int64_t)(f0 + row) * L, (int64_t)z.trow0[t] + row, col);
   }
 }
 
@@ -151,6 +184,7 @@ __global__ __launch_bounds__(256) void k_pp(Tab z, const double* __restrict__ x,
         d[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[q / 2][q % 2], xv[q][u / 2][u % 2], d[u], 0, 0, 0);
   }
   const int nr = cst(z.tnr)[t], f0 = cst(z.tfirst)[t];
+  uint32_t out = take_out(d);
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int row = 4 * lk + i;
@@ -163,12 +197,19 @@ __global__ __launch_bounds__(256) void k_pp(Tab z, const double* __restrict__ x,
       }
     }
   }
+  for (; out; out &= out - 1) {
+    const int q = __builtin_ctz(out), row = 4 * lk + (q >> 2), h = q >> 1 & 1;
+    const int at = h ? c[1] : c[0], col = (h ? cl[1] : cl[0]) + (q & 1);
+    if (row < nr && col >= at && col < L)
+      again(z, x, y + sec + (int64_t)(f0 + row) * L, (int64_t)z.trow0[t] + row, col);
+  }
 }
 
 // NN: a tile of 8 proton rows staged in LDS (16-byte pieces of a column's 8
 // values, one array a piece, so that neighbouring columns are neighbours), one
 // read of a column's entry (source column, value) serves all of them.  FP64
-// stages 2,048 source columns at a time.
+// stages 2,048 source columns at a time.  Each half of a row has a column of
+// zeros before it, which the padding entries name: no padding reads an amplitude.
 template <typename T>
 __global__ __launch_bounds__(1024) void k_nn(Tab z, const T* __restrict__ x, T* __restrict__ y, int accumulate) {
   constexpr int R = kNnRows, V = 16 / (int)sizeof(T), NA = R / V;  // values a piece, pieces
@@ -183,20 +224,29 @@ __global__ __launch_bounds__(1024) void k_nn(Tab z, const T* __restrict__ x, T* 
   const int f0 = cst(z.nf0)[t], nr = cst(z.nnr)[t];
   const int cn = cst(z.pconj)[cst(z.psec)[f0]];
   const int L = cst(z.nlen)[cn], ncc = (L + 63) >> 6;
-  const int cs = min(L, C);  // staged columns (stride of the pieces)
+  // places of staged columns and zeros (stride of the pieces)
+  const int cs = sizeof(T) == 4 ? L + 1 + (L > 2048) : min(L, C) + 1;
   const int64_t base = cst(z.pstart)[f0];
   constexpr int Q = 4;  // column chunks of a wave (rows up to 4096 columns)
   for (int h = 0; h < (sizeof(T) == 8 ? 2 : 1); h++) {
     const int h0 = h * C;
     if (h0 >= L) break;
     if (h) __syncthreads();
+    if (tid < NA) {
+      Piece u;
+#pragma unroll
+      for (int i = 0; i < V; i++) u.v[i] = T(0);
+      xs[tid * cs] = u;
+      if (sizeof(T) == 4 && L > 2048) xs[tid * cs + 2049] = u;
+    }
     for (int c = tid; c < min(C, L - h0); c += blockDim.x) {
+      const int at = c + 1 + (sizeof(T) == 4 && c >= 2048);
 #pragma unroll
       for (int p = 0; p < NA; p++) {
         Piece u;
 #pragma unroll
         for (int i = 0; i < V; i++) u.v[i] = p * V + i < nr ? x[base + (int64_t)(p * V + i) * L + h0 + c] : T(0);
-        xs[p * cs + c] = u;
+        xs[p * cs + at] = u;
       }
     }
     __syncthreads();
@@ -241,7 +291,7 @@ __global__ __launch_bounds__(1024) void k_nn(Tab z, const T* __restrict__ x, T* 
           for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int k = 0; k < NA; k++) {
-              const Piece e = xs[k * cs + (sizeof(T) == 4 ? hh * 2048 : 0) + col[i]];
+              const Piece e = xs[k * cs + (sizeof(T) == 4 ? hh * 2049 : 0) + col[i]];
 #pragma unroll
               for (int j = 0; j < V; j++) a[k * V + j] = fma(u[i], e.v[j], a[k * V + j]);
             }
@@ -325,7 +375,7 @@ void apply_t(const Owner& o, const T* x, T* y, int accumulate, hipStream_t st) {
   else z.pA64 = o.pA64, z.nval64 = o.nval64;
   constexpr int C = sizeof(T) == 4 ? 4096 : 2048;
   const int nw = std::min(16, (o.lmax + 63) / 64);
-  const size_t lds = (size_t)std::min(o.lmax, C) * kNnRows * sizeof(T);
+  const size_t lds = (size_t)(std::min(o.lmax, C) + 2) * kNnRows * sizeof(T);
   hipLaunchKernelGGL(k_nn<T>, dim3((o.t.nnn + 255) / 256 * 256), dim3(64 * nw), lds, st, z, x, y, accumulate);
   HIP_OK(hipGetLastError());
   if (o.t.npp > 0) {
@@ -444,12 +494,12 @@ bool structure(Owner& o, const Host& g, hipStream_t st) {
         const size_t o0 = nsrc.size() / 64;
         if (o0 >= (1u << 22)) return false;
         nng[((size_t)c * 64 + cc) * 2 + h] = (uint32_t)o0 << 10 | (uint32_t)np;
-        // padding entries: value zero at the chunk's first source column
+        // padding entries: value zero at the column of zeros
         nsrc.resize(nsrc.size() + (size_t)np * 64, 0u);
         for (int l = 0; l < nl; l++)
           for (int64_t q = lo[l]; q < hi[l]; q++) {
             const int i = (int)(q - lo[l]);
-            const uint32_t sc = (uint32_t)(t.tb[1].src[q] - N.secfirst[c]) - 2048u * h;
+            const uint32_t sc = (uint32_t)(t.tb[1].src[q] - N.secfirst[c]) - 2048u * h + 1u;
             nsrc[(o0 + i / 2) * 64 + l] |= sc << (16 * (i % 2));
           }
       }
@@ -473,7 +523,10 @@ bool structure(Owner& o, const Host& g, hipStream_t st) {
   d.pstart = g.pstart;
   d.nng = put(o, nng, st);
   d.nsrc = put(o, nsrc, st);
-  o.row0 = put(o, row0, st);
+  d.trow0 = put(o, row0, st);
+  d.pp_ptr = g.pp_ptr;
+  d.pp_src = g.pp_src;
+  d.pp_val = g.pp_val;
   o.usrc = put(o, usrc, st);
   o.blocks = tblk.back();
   o.nrows = (int64_t)nsrc.size() / 64;
@@ -493,9 +546,9 @@ void values(Owner& o, const Host& g, const T** pA, const T** nval, hipStream_t s
   T* A = get<T>(o, na);
   HIP_OK(hipMemsetAsync(A, 0, na * sizeof(T), st));
   if constexpr (sizeof(T) == 4)
-    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.row0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, A, nullptr);
+    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.t.trow0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, A, nullptr);
   else
-    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.row0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, nullptr, A);
+    k_pp_fill<<<o.ntile, 256, 0, st>>>(o.ntile, o.t.trow0, o.t.tnr, o.t.tblk, o.usrc, g.pp_ptr, g.pp_src, g.pp_val, nullptr, A);
   HIP_OK(hipGetLastError());
   std::vector<T> v((size_t)o.nrows * 128, T(0));
   int64_t lo[64], hi[64];

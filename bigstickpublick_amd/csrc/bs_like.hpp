@@ -26,6 +26,10 @@ struct Tab {
   const uint32_t* psrc;       // [block][k % 4][k / 4]: source row's offset within the sector
   const float* pA32;          // [block][lane][step]: see k_pp
   const double* pA64;         // [block][step / 2][lane][step % 2]
+  const int32_t* trow0;       // [tile] first proton SD
+  const int64_t* pp_ptr;      // the entries by proton SD
+  const int32_t* pp_src;
+  const double* pp_val;
   // NN
   const int32_t* nf0;         // [tile] first proton row
   const int32_t* nnr;         // [tile] rows
@@ -35,8 +39,8 @@ struct Tab {
   const int64_t* pstart;
   // entries of column chunk cc of neutron sector c, source columns below 2048
   // (h = 0) and from 2048 on (h = 1, counted from there): g = nng[(c * 64 + cc) *
-  // 2 + h], rows of 64 words (two entries' source columns) from row g >> 10,
-  // (g & 1023) of them (an even number); values [2 row + entry][64]
+  // 2 + h], rows of 64 words (two entries' source columns, each plus one; 0: none)
+  // from row g >> 10, (g & 1023) of them (an even number); values [2 row + entry][64]
   const uint32_t* nng;
   const uint32_t* nsrc;
   const float* nval32;
@@ -51,7 +55,6 @@ struct Owner {
   const double *pA64 = nullptr, *nval64 = nullptr;
   int ntile = 0;                // PP tiles, their first rows and sources, for the values
   int64_t blocks = 0, nrows = 0;
-  const int32_t* row0 = nullptr;
   const int32_t* usrc = nullptr;
   std::vector<uint32_t> nng;
   std::vector<void*> mem;
