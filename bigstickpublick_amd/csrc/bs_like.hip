@@ -1,11 +1,10 @@
 // bs_like.hip -- proton-proton and neutron-neutron parts of H x on large bases.
 #include "bs_like.hpp"
+#include "bs_parallel.hpp"
 
 #include <algorithm>
-#include <atomic>
 #include <stdexcept>
 #include <string>
-#include <thread>
 
 namespace bsl {
 namespace {
@@ -354,19 +353,6 @@ V* put(Owner& o, const std::vector<V>& v, hipStream_t st) {
   return p;
 }
 
-template <typename F>
-void parallel(int n, F&& body) {
-  std::atomic<int> next(0);
-  auto work = [&]() {
-    for (int i = next++; i < n; i = next++) body(i);
-  };
-  const int nt = (int)std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency()));
-  std::vector<std::thread> th;
-  for (int i = 1; i < std::min(nt, n); i++) th.emplace_back(work);
-  work();
-  for (auto& q : th) q.join();
-}
-
 template <typename T>
 void apply_t(const Owner& o, const T* x, T* y, int accumulate, hipStream_t st) {
   if (!o.ok[sizeof(T) == 4 ? 0 : 1]) throw std::runtime_error("like-particle tables missing");
@@ -440,7 +426,7 @@ bool structure(Owner& o, const Host& g, hipStream_t st) {
   }
   const int nt = (int)row0.size();
   std::vector<std::vector<int32_t>> uni(nt);
-  parallel(nt, [&](int i) {
+  bs::parallel(nt, [&](int i) {
     std::vector<int32_t>& u = uni[i];
     const int64_t a = t.tb[0].rowptr[row0[i]], b = t.tb[0].rowptr[row0[i] + tnr[i]];
     u.assign(t.tb[0].src.begin() + a, t.tb[0].src.begin() + b);
