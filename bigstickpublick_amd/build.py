@@ -3,6 +3,7 @@
 import os
 import shutil
 import subprocess
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -29,17 +30,22 @@ def build_native(verbose=False):
     for src in SOURCES:
         obj = os.path.join(bdir, src + ".o")
         cmd = [HIPCC] + [f for f in HIP_FLAGS if f != "-shared"] + inc + ["-c", os.path.join(CSRC, src), "-o", obj]
-        jobs.append((obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-    for obj, p in jobs:
-        out = p.communicate()[0]
+        log = tempfile.TemporaryFile(mode="w+")  # (a full pipe would stop the compiler)
+        jobs.append((src, obj, log, subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT)))
+    failed = []
+    for src, obj, log, p in jobs:
+        p.wait()
+        log.seek(0)
+        out = log.read()
+        log.close()
         if p.returncode != 0:
-            for _, q in jobs:
-                q.wait()
-            raise RuntimeError("hipcc failed:\n" + out)
-        if verbose:
+            failed.append("%s:\n%s" % (src, out))
+        elif verbose:
             print(out)
+    if failed:
+        raise RuntimeError("hipcc failed:\n" + "\n".join(failed))
     tmp = LIB + ".tmp"
-    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-o", tmp] + [obj for obj, _ in jobs] +
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-o", tmp] + [j[1] for j in jobs] +
                        ["-lrocsolver", "-lrocblas"], capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("hipcc failed:\n" + r.stdout + r.stderr)
