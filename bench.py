@@ -88,30 +88,44 @@ def traffic_from_profiles(variant):
     return None
 
 
+# the kernels of one H x: the tile kernel, and before it the NN and PP kernels of the
+# variants that take those parts apart (prefetch 2)
+H_KERNELS = (("tiles", r"\bk_apply_tiles<float"), ("nn", r"\bk_nn<float>"), ("pp", r"\bk_pp\(.*float const"))
+
+
 def traffic_from_dbs(fetch_db, write_db, D):
-    """Per-dispatch FETCH_SIZE / WRITE_SIZE (KiB) of the H x kernel, scaled by
-    what the same counters read for the copy probe (one plain copy of 4*D
+    """FETCH_SIZE / WRITE_SIZE (KiB) of one H x, its kernels together, scaled
+    by what the same counters read for the copy probe (one plain copy of 4*D
     bytes read and 4*D written, the last copy dispatch of the run)."""
+    import re
     import sqlite3
     out = {}
     for key, db in (("fetch", fetch_db), ("write", write_db)):
         c = sqlite3.connect(db)
         rows = list(c.execute("select dispatch_id, kernel_name, value, duration from counters_collection "
                               "order by dispatch_id"))
-        kern = [r for r in rows if "k_apply_tiles<float" in r[1]]
         copies = [r for r in rows if "copy" in r[1].lower() and r[2] > 1e5]
-        if not kern or not copies:
+        parts = {}
+        for part, pattern in H_KERNELS:
+            kern = [r for r in rows if re.search(pattern, r[1])]
+            if len(set(r[1] for r in kern)) > 1:
+                raise RuntimeError("several H x kernels in %s (run with --variant)" % db)
+            if kern:
+                parts[part] = kern
+        if "tiles" not in parts or not copies:
             raise RuntimeError("no H x or copy-probe dispatch in " + db)
-        names = sorted(set(r[1] for r in kern))
-        if len(names) != 1:
-            raise RuntimeError("several H x kernels in %s (run with --variant)" % db)
+        n = len(parts["tiles"])
+        if any(len(k) != n for k in parts.values()) or len(parts) == 2:
+            raise RuntimeError("not every H x in %s has the same kernels" % db)
         probe = copies[-1]
         scale = 4.0 * D / (probe[2] * 1024.0)
-        vals = [r[2] for r in kern]
+        vals = [sum(k[i][2] for k in parts.values()) for i in range(n)]
         out[key] = {"kib_raw": vals, "probe_kib": probe[2], "probe_kernel": probe[1], "scale": scale,
-                    "bytes_per_launch": sum(vals) / len(vals) * 1024.0 * scale,
-                    "mean_duration_ns": sum(r[3] for r in kern) / len(kern)}
-        out["kernel"] = names[0]
+                    "kib_raw_by_kernel": {p: sum(r[2] for r in k) / n for p, k in parts.items()},
+                    "bytes_per_launch": sum(vals) / n * 1024.0 * scale,
+                    "mean_duration_ns": sum(r[3] for k in parts.values() for r in k) / n}
+        out["kernel"] = parts["tiles"][0][1]
+        out["kernels"] = [k[0][1] for k in parts.values()]
     out["bytes_per_launch"] = out["fetch"]["bytes_per_launch"] + out["write"]["bytes_per_launch"]
     return out
 
@@ -229,7 +243,7 @@ def block_leg(s, K, steps, warmup, g):
     torch.cuda.empty_cache()
     return {"K": K, "kernel_ms": ms, "hv_per_s_per_vector": K * 1000.0 / ms, "variant": chosen,
             "autotune_ms": {str(v): round(float(t), 3) for v, t in enumerate(tms) if t > 0},
-            "what": "0 = one wave per state, 1-4 = one proton row per workgroup, 5-6 = two-row tiles"}
+            "what": "0 = staged jumps of a row or one wave per state, 1-4 = one proton row per workgroup, 5-6 = two-row tiles"}
 
 
 def batch_leg(sps, case, K, steps, warmup, solve, max_restarts, work, n_ops):
@@ -432,7 +446,7 @@ def main():
         m = re.search(r"k_apply_tiles<float, 512, (\d+), (\d+), (\d+), (true|false)>", t["kernel"])
         t["workload"] = "%s M=0 D=%d FP32" % (case.name, s.dim)
         t["variant"] = [int(m.group(2)), int(m.group(3)), a.variant if a.variant >= 0 else None,
-                        int(m.group(4) == "true")]
+                        2 if len(t["kernels"]) > 1 else int(m.group(4) == "true")]
         if a.variant >= 0:
             t["variant"] = list(System.variants()[a.variant])
         old = {"variants": []}
@@ -540,7 +554,8 @@ def main():
         "setup_s": {"host_tables": t_host, "upload": t_upload, "autotune": t_tune},
         "autotune_ms": {"R%d_G%d_xcd%d_pf%d" % v: round(float(t), 3)
                         for v, t in zip(System.variants(), s.autotune_times("f32")) if t > 0},
-        "traffic_source": os.path.relpath(TRAFFIC_JSON, ROOT) if traffic else None,
+        "traffic_source": os.path.relpath(TRAFFIC_JSON, ROOT) if traffic else
+                          "none: %s has no counters of this variant" % os.path.relpath(TRAFFIC_JSON, ROOT),
         "kernel_variant": {"rows_per_tile": System.variants()[variant][0],
                            "staged_rows": System.variants()[variant][1],
                            "xcd_map": System.variants()[variant][2],
