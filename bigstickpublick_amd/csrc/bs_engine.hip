@@ -3879,7 +3879,7 @@ int run_lanczos(bs_system* s, const bs_lanczos_params* p, double* alpha_out, dou
     V.alloc((size_t)mtot * ld);
     w.alloc(D);
     part.alloc((size_t)nb * mtot);
-    dots.alloc(mtot);
+    dots.alloc(std::max(mtot, 3));  // (the polish has three)
     ab.alloc(2 * (size_t)mtot + 4);  // alpha[0..], beta[mtot..], then the first flagged step (an int)
   }
   double* d_alpha = ab.p;
