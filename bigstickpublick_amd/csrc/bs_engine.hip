@@ -1374,7 +1374,7 @@ __global__ __launch_bounds__(256) void k_density_nn_g(DevTables tb, DensTables d
 // behind the row), whose values it reads from the row staged in LDS, for four
 // v_mfma_f64_16x16x4.  Nothing is summed across lanes, where one list a
 // (jump, operator) cost 24 shuffles for some 80 products: pf 4p4n FP32 2.87 ->
-// 0.50 ms.
+// 0.69 ms (of a gradient's 1.32; the matrix cores are busy for half of it).
 typedef double dens_d4 __attribute__((ext_vector_type(4)));
 template <typename T>
 __global__ __launch_bounds__(256) void k_density_pn(DevTables tb, DensTables dn, const T* __restrict__ x,
@@ -3563,12 +3563,12 @@ void want_tables(bs_system* s, bool named = false) {
   std::lock_guard<std::mutex> lock(s->want);
   if (done()) return;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  HIP_OK(hipThreadExchangeStreamCaptureMode(&mode));
   hipStream_t st = nullptr;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
   try {
     HIP_OK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     const std::vector<int32_t> nlen = s->nlen.download(st);
-    if (!s->brief_tried && *std::max_element(nlen.begin(), nlen.end()) <= bss::kMaxRow) {
+    if (!s->brief_tried && s->dt.lmax <= bss::kMaxRow) {
       const std::vector<int32_t> f0[3] = {s->tile_f0[0].download(st), s->tile_f0[1].download(st), s->tile_f0[2].download(st)};
       const std::vector<int32_t> nr[3] = {s->tile_nr[0].download(st), s->tile_nr[1].download(st), s->tile_nr[2].download(st)};
       const std::vector<int64_t> pp[3] = {s->tpp_ptr[0].download(st), s->tpp_ptr[1].download(st), s->tpp_ptr[2].download(st)};
@@ -3586,7 +3586,7 @@ void want_tables(bs_system* s, bool named = false) {
     if (!s->brief_tried) s->brief.release();
   }
   if (st) (void)hipStreamDestroy(st);
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
   s->brief_tried.store(true, std::memory_order_release);
   if (like) s->like_tried[di].store(true, std::memory_order_release);
 }

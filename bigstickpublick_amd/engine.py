@@ -363,7 +363,8 @@ class System:
 
     def lanczos(self, nkeep, niter, thick=0, max_restarts=0, dtype="f32", tol=0.0, polish=True,
                 want_vectors=False, conv_test=1, ncheck_ex=0, target=None, target_test="reference"):
-        """Lanczos from the uniform pivot.  With tol > 0 the run stops by the
+        """Lanczos from the uniform pivot; autotune(dtype) first for speed
+        (until then the largest tile runs).  With tol > 0 the run stops by the
         reference's test conv_test (0: mean energy change, 1: largest energy
         change, 2 / 3: mean / largest change of the Ritz vectors)
         over nkeep + ncheck_ex Ritz values (the reference's ld is conv_test=0,

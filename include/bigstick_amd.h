@@ -135,7 +135,11 @@ int bs_apply_h(bs_system *sys, const void *x, void *y, int dtype, int accumulate
  * dtype; bs_set_variant forces one (-1 = default choice).  FP32 steps of
  * bs_lanczos, bs_lanczos_noalloc and bs_strength add a column's products in an
  * order that the space's sizes fix, and take the fastest variant of that order,
- * or the forced one: a run's unconverged Ritz vectors follow the order. */
+ * or the forced one: a run's unconverged Ritz vectors follow the order.  Until
+ * bs_autotune or bs_set_variant, solves of either dtype take the largest tile;
+ * bs_apply_h builds the tables of prefetch 2 to 5 in its first call (which waits
+ * for that; under stream capture it takes the largest tile) and uses the shape
+ * that is usually the fastest. */
 int bs_num_variants(int *n);
 int bs_variant_info(int variant, int *rows, int *staged, int *xcd_map, int *prefetch);
 int bs_set_variant(bs_system *sys, int dtype, int variant);
