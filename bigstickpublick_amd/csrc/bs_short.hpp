@@ -9,7 +9,9 @@
 
 namespace bss {
 
-constexpr int kMaxRow = 576;             // longest neutron row
+// Longest neutron row: nine 64-column chunks (pf rows of four neutrons have up to 565
+// SDs, of five 1,651, which the tile kernel takes).
+constexpr int kMaxRow = 576;
 constexpr int kMaxChain = 256;           // the same for the ordered shapes
 // Shapes below kSplit share a column's sum among waves; the next two (FP32) keep its
 // order.
