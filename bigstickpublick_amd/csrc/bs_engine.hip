@@ -3665,7 +3665,7 @@ int settle(float* times, int n, float best, int bestv, hipEvent_t e0, hipEvent_t
   float least = 1e30f;
   for (int v = 0; v < n; v++) {
     if (!close(v)) continue;
-    constexpr int kTimes = 8;
+    constexpr int kTimes = 4;
     HIP_OK(hipEventRecord(e0, st));
     for (int i = 0; i < kTimes; i++) launch(v);
     HIP_OK(hipEventRecord(e1, st));
@@ -4811,23 +4811,17 @@ struct Timer {
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
   }
-  // ms of the second of two launches; of short ones, which vary by a tenth, the least
-  // of the four after the first
+  // ms of one launch (the second of two where it is new)
   template <typename F>
-  float once(F&& launch) {
+  float once(F&& launch, bool first = true) {
+    if (first) launch(x.p, y.p);
+    HIP_OK(hipEventRecord(e0, nullptr));
     launch(x.p, y.p);
-    float least = 1e30f;
-    for (int i = 0; i < 4; i++) {
-      HIP_OK(hipEventRecord(e0, nullptr));
-      launch(x.p, y.p);
-      HIP_OK(hipEventRecord(e1, nullptr));
-      HIP_OK(hipEventSynchronize(e1));
-      float ms = 0.0f;
-      HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-      least = std::min(least, ms);
-      if (least > 0.1f) break;
-    }
-    return least;
+    HIP_OK(hipEventRecord(e1, nullptr));
+    HIP_OK(hipEventSynchronize(e1));
+    float ms = 0.0f;
+    HIP_OK(hipEventElapsedTime(&ms, e0, e1));
+    return ms;
   }
 };
 
@@ -4843,30 +4837,41 @@ int batch_variant(bs_system* s, const BatchVals& bv) {
   const int key = multi_key<T>(bv);
   auto it = s->multi_choice.find(key);
   if (it != s->multi_choice.end()) return it->second;
-  want_lanes(s, bv.K, (int)sizeof(T));
-  Timer<T> tm(s->t.dim * bv.K);
-  float best = 1e30f;
-  int bestv = 0;
-  std::array<float, 8> ms{};
-  for (int v = 0; v < kNumMulti; v++) {
-    if (!multi_fits(s, v, bv.K, sizeof(T), bv.vk == 0)) continue;
-    if (v == 0 && s->tiles_ok && s->t.dim > kPerStateDim) continue;
-    ms[v] = tm.once([&](const T* x, T* y) { launch_batched_v<T>(s, v, bv, x, y, nullptr); });
-    if (ms[v] < best) { best = ms[v]; bestv = v; }
-  }
   // Variant 0 has two kernels of the same bits.  A workgroup of k_apply_lanes takes a
   // proton row: with few rows most CUs have none (pf 1p4n, 20 rows, K = 34: 1,732 us,
   // per state 207; sd 1p6n, 12 rows, K = 12: 109 and 40), with short ones a wave has no
-  // columns (pf 7p1n, rows of 1 to 4, K = 3: 6.97 ms and 3.33).  There the per-state
-  // kernel is timed too; with rows for three quarters of the CUs, of 16 columns on
-  // average, it took 1.4 to 10 times as long in every one of 60 batches and blocks, and
-  // twice to 70 times as long as the tiles.
-  float per_state = 0.0f;
-  if (ms[0] > 0.0f && !(s->dt.nP >= 192 && s->t.dim >= (int64_t)16 * s->dt.nP)) {
-    per_state = tm.once([&](const T* x, T* y) { launch_per_state<T>(s, bv, x, y, nullptr); });
-    s->multi_per_state[key] = per_state < ms[0];
-    ms[0] = std::min(ms[0], per_state);
-    if (ms[0] < best) { best = ms[0]; bestv = 0; }
+  // columns (pf 7p1n, rows of 1 to 4, K = 3: 6.97 ms and 3.33): below 128 rows, or 4
+  // columns on average, it won by a tenth at most and is left out.  With rows for three
+  // quarters of the CUs, of 16 columns on average, the per-state kernel took 1.4 to 10
+  // times as long in every one of 60 batches and blocks, and twice to 70 times as long as
+  // the tiles, and is left out.  Between, both are timed.
+  const int64_t rows = s->dt.nP;
+  const bool few = rows < 128 || s->t.dim < 4 * rows, many = rows >= 192 && s->t.dim >= 16 * rows;
+  if (!few) want_lanes(s, bv.K, (int)sizeof(T));
+  const bool lanes = !few && s->lane_ok && lane_shape(s, bv.K, (int)sizeof(T)).H;
+  Timer<T> tm(s->t.dim * bv.K);
+  float best = 1e30f, per_state = 0.0f;
+  int bestv = 0;
+  std::array<float, 8> ms{};
+  auto state = [&](const T* x, T* y) { launch_per_state<T>(s, bv, x, y, nullptr); };
+  auto lane = [&](const T* x, T* y) { launch_lanes<T>(s, bv, x, y, nullptr); };
+  for (int v = 0; v < kNumMulti; v++) {
+    if (!multi_fits(s, v, bv.K, sizeof(T), bv.vk == 0)) continue;
+    if (v > 0) {
+      ms[v] = tm.once([&](const T* x, T* y) { launch_batched_v<T>(s, v, bv, x, y, nullptr); });
+    } else if (s->tiles_ok && s->t.dim > kPerStateDim) {
+      continue;
+    } else {
+      if (lanes) ms[0] = tm.once(lane);
+      if (!lanes || !many) per_state = tm.once(state);
+      for (int i = 0; lanes && per_state > 0.0f && i < 3 && per_state < 1.3f * ms[0] && ms[0] < 1.3f * per_state && ms[0] < 0.2f; i++) {
+        ms[0] = std::min(ms[0], tm.once(lane, false));  // (short launches vary by a tenth)
+        per_state = std::min(per_state, tm.once(state, false));
+      }
+      s->multi_per_state[key] = !lanes || (per_state > 0.0f && per_state < ms[0]);
+      if (s->multi_per_state[key]) ms[0] = per_state;
+    }
+    if (ms[v] < best) { best = ms[v]; bestv = v; }
   }
   s->multi_once[key] = ms;
   s->multi_once[key][0] = per_state;
